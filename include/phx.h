@@ -628,7 +628,12 @@ typedef struct {
                                            only), set up by phx_engine_reset */
     int32_t sc_stage_shape[PHX_MAX_SC_STAGES + 1];  /* PHX_SHAPE_* of stages
                                            1..sc_stages (entry 0 unused) */
-    int32_t pad_sc2;
+    int32_t ahead;                      /* 1: every turn of a launch sequence
+                                           runs the same program and no wake
+                                           kick acts on dp (0 is always
+                                           valid).  The particle pass may then
+                                           form the z sums of the next turn
+                                           (see phx_engine_turns) */
 } phx_engine;
 
 /* stats row r (state after r turns, r = 0 .. turns run) holds 33 FP64 sums
@@ -659,7 +664,15 @@ int phx_engine_reset(const phx_engine *e, phx_stream_t stream);
    entry) and the wake convolution; without a wake field, the pass and a
    one-block finalize; one more launch ahead of the first turn records
    particle 0 (phx_engine_snapshot).  The wake kick of the last turn stays
-   pending until phx_engine_flush. */
+   pending until phx_engine_flush.
+   With e->ahead set (and dipolar or plates kicks, no space charge, the
+   slices' histogram within the LDS), sequences of PHX_AHEAD_MIN_TURNS or
+   more turns are three launches per turn: the pass knows its turn's cuts
+   when it starts, slices the particles it has just moved, and sums the next
+   turn's z (the longitudinal motion alone fixes it) for the next turn's
+   cuts, which the merge folds.  Two launches ahead of the first turn give
+   its cuts.  The results are those of the four-launch turn bit for bit. */
+#define PHX_AHEAD_MIN_TURNS 4
 int phx_engine_turns(const phx_engine *e, int32_t n_turns, phx_stream_t stream);
 /* Applies a pending wake kick (and records the final statistics row). */
 int phx_engine_flush(const phx_engine *e, phx_stream_t stream);
@@ -667,13 +680,16 @@ int phx_engine_flush(const phx_engine *e, phx_stream_t stream);
    merge, 2 wake convolution (stages 1-2 need a wake field).  Running 0, 1, 2
    in order is one turn; used to time the stages separately.  Call
    phx_engine_snapshot before the first stage 0 after the coordinates
-   changed outside the engine. */
+   changed outside the engine.  Stages 3, 4, 5 are those of the three-launch
+   turn (pass and slicing, merge, convolution) where it applies, else stages
+   0, 1, 2: after phx_engine_snapshot and only stages 3, 4, 5 since. */
 int phx_engine_stage(const phx_engine *e, int32_t stage, phx_stream_t stream);
 /* Records particle 0's coordinates in the workspace: the shifts of the
    shifted sums of the next particle pass (stats.pyx:cov takes the first
    particle), read there by every block while block 0 rewrites particle 0.
    phx_engine_turns and phx_engine_flush call it themselves; graph replays
-   do not. */
+   do not.  Where three-launch turns apply (phx_engine_turns), it also forms
+   the cuts of the next turn. */
 int phx_engine_snapshot(const phx_engine *e, phx_stream_t stream);
 
 /* Allocation-free variant of phx_engine_turns.  It has no counterpart in

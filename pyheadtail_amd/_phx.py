@@ -189,7 +189,7 @@ class Engine(C.Structure):
                 ("kicks", C.c_void_p), ("counts", C.c_void_p),
                 ("slice_means", C.c_void_p), ("ws", C.c_void_p),
                 ("sc_slices", C.c_int32), ("pad_sc", C.c_int32), ("sc_ws", C.c_void_p),
-                ("sc_stage_shape", C.c_int32 * (MAX_SC_STAGES + 1)), ("pad_sc2", C.c_int32)]
+                ("sc_stage_shape", C.c_int32 * (MAX_SC_STAGES + 1)), ("ahead", C.c_int32)]
 
 
 RECORDS = {

@@ -143,7 +143,7 @@ void stage_blocks(const EngineArgs &a, int (&nb)[BS_COUNT]) {
   nb[BS_CUTS] = 1;
   nb[BS_HIST] = hist_blocks(e.n);
   const bool has_wake = S > 0 && a.n_kicks > 0;
-  nb[BS_MERGE] = (S + merge_sl(S) - 1) / merge_sl(S) + (has_wake && engine_has_rw(e) ? 1 : 0);
+  nb[BS_MERGE] = merge_blocks(S, merge_sl(S), has_wake && engine_has_rw(e), false, false);
   nb[BS_CONV] = (ck == 0 || (ck & PHX_CONV_GENERAL)) ? (S + WK_TILE - 1) / WK_TILE * a.n_kicks * a.T : 0;
   nb[BS_RW] = (ck == 0 || (ck & PHX_CONV_RW_DOT)) ? rw_tiles * conv_rows(S, a.T) : 0;
   nb[BS_RWMF] = (ck == 0 || (ck & PHX_CONV_RW_MFMA)) ? rw_tiles * conv_rows(S, a.T) : 0;

@@ -1,7 +1,12 @@
 // Device-side building blocks shared by the standalone element kernels and
 // the fused turn engine.  Everything here is FP64 and is compiled with
 // -ffp-contract=off so that each arithmetic operation is one IEEE-754
-// rounding, in the order the reference's NumPy expressions evaluate them.
+// rounding.  Slicing, the linear map and the transverse map without detuning
+// are the operations of the reference's NumPy expressions in their order.
+// Where a sine or cosine enters (RF kicks, detuned phases), which no two
+// libraries round alike, the expressions are arranged for fewer operations:
+// phases in turns, constant quotients folded once, sums of products as FMAs,
+// with fewer roundings than the reference's order.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -100,6 +105,27 @@ __device__ __forceinline__ double slice_floor_r(double z, double tail, double wi
   return floor(div_rcp(z - tail, width, inv_width));
 }
 
+// The slices of one state for many particles: index(z) is the slice of z in
+// [0, S), or a negative number outside the cuts; int32(floor((z - tail) /
+// width)) exactly.  For widths in [2^-400, 2^400] the quotient is div_rcp's
+// without its range check: a quotient of extreme magnitude only has to keep
+// its sign and its place beyond S, and a non-finite one becomes NaN, which is
+// outside either way.  Other widths (uniform) divide.
+struct SliceBins {
+  double tail, width, inv, S;
+  bool plain;
+  __device__ __forceinline__ SliceBins() {}
+  __device__ __forceinline__ SliceBins(double t, double w, int n)
+      : tail(t), width(w), inv(1.0 / w), S((double)n), plain(w >= 0x1p-400 && w <= 0x1p400) {}
+  __device__ __forceinline__ int index(double z) const {
+    const double a = z - tail;
+    const double q0 = a * inv;
+    double q = fma(fma(-q0, width, a), inv, q0);
+    if (__builtin_expect(!plain, 0)) q = a / width;
+    return q >= 0.0 && q < S ? (int)q : -1;
+  }
+};
+
 __device__ __forceinline__ int32_t x86_cvt_i32(double f) {
   // cvttsd2si semantics: NaN and out-of-range values give INT32_MIN
   if (!(f >= -2147483648.0 && f < 2147483648.0)) return INT32_MIN;
@@ -110,62 +136,74 @@ __device__ __forceinline__ int32_t x86_cvt_i32(double f) {
 // Transverse segment map (trackers/transverse_tracking.py:138-196) with the
 // detuners (trackers/detuners.py:64-98 chromaticity, :128-151 amplitude).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void detune_amplitude(const phx_detuner &d, const P6 &p, double &qx,
-                                                 double &qy) {
-  // Jx = 1/2*((1+a^2)/b*x**2 + 2*a*x*xp + b*xp**2)
-  const double jx = 0.5 * ((d.gx * (p.x * p.x) + (d.ax2 * p.x) * p.xp) + d.bx * (p.xp * p.xp));
-  const double jy = 0.5 * ((d.gy * (p.y * p.y) + (d.ay2 * p.y) * p.yp) + d.by * (p.yp * p.yp));
-  qx = div_rcp(d.dapp_x * jx + d.dapp_xy * jy, d.p0, d.inv_p0);
-  qy = div_rcp(d.dapp_y * jy + d.dapp_yx * jx, d.p0, d.inv_p0);
-}
-
-__device__ __forceinline__ void detune(const phx_detuner &d, const P6 &p, double &qx,
-                                       double &qy) {
-  if (d.type == PHX_DET_CHROMA) {
-    // Horner form of (c0 + (c1 + c2*dp)*dp)*dp, the same association as the
-    // explicit order-1..3 polynomials and np.polynomial.polyval.
-    double ax = d.cx[d.order - 1], ay = d.cy[d.order - 1];
-    for (int i = d.order - 2; i >= 0; --i) {
-      ax = d.cx[i] + ax * p.dp;
-      ay = d.cy[i] + ay * p.dp;
+// A tune shift added to the phases (in turns) of N particles.
+//   chromaticity: Horner form of (c0 + (c1 + c2 dp) dp) dp;
+//   amplitude: dQ_x = (dapp_x Jx + dapp_xy Jy) / p0 with
+//   Jx = ((1 + a^2)/b x^2 + 2 a x xp + b xp^2) / 2; the strengths come with
+//   1 / (2 p0) folded in.
+// SMOOTH: segments (PHX_DETS_SMOOTH) with alpha = 0, for which the host
+// checked ax2 = ay2 = 0 and gx, gy > 0: then (ax2 x) xp is a zero added to
+// bx xp^2 >= +0, which leaves it unchanged, and the term is dropped (the same
+// bits for finite coordinates).
+template <int N, bool SMOOTH = false>
+__device__ __forceinline__ void detune_amplitude_n(const phx_detuner &d, const P6 (&p)[N],
+                                                   double (&ux)[N], double (&uy)[N]) {
+  const double f = 0.5 * d.inv_p0;
+  const double axx = d.dapp_x * f, axy = d.dapp_xy * f, ayy = d.dapp_y * f, ayx = d.dapp_yx * f;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    double jx = (d.bx * p[k].xp) * p[k].xp, jy = (d.by * p[k].yp) * p[k].yp;
+    if constexpr (!SMOOTH) {
+      jx = fma(d.ax2 * p[k].x, p[k].xp, jx);
+      jy = fma(d.ay2 * p[k].y, p[k].yp, jy);
     }
-    qx = ax * p.dp;
-    qy = ay * p.dp;
-  } else {
-    detune_amplitude(d, p, qx, qy);
+    jx = fma(d.gx * p[k].x, p[k].x, jx);
+    jy = fma(d.gy * p[k].y, p[k].y, jy);
+    ux[k] = ux[k] + fma(axx, jx, axy * jy);
+    uy[k] = uy[k] + fma(ayy, jy, ayx * jx);
   }
 }
 
-// Smooth segments (PHX_DETS_SMOOTH) have alpha = 0, and the host sets the
-// flag only with ax2 = ay2 = 0 and gx, gy > 0: then (ax2 x) xp is a zero
-// added to gx x^2 >= +0, which leaves it unchanged, and the term is dropped
-// (the same bits for finite coordinates).
-__device__ __forceinline__ void detune_amplitude_smooth(const phx_detuner &d, const P6 &p,
-                                                        double &qx, double &qy) {
-  const double jx = 0.5 * (d.gx * (p.x * p.x) + d.bx * (p.xp * p.xp));
-  const double jy = 0.5 * (d.gy * (p.y * p.y) + d.by * (p.yp * p.yp));
-  qx = div_rcp(d.dapp_x * jx + d.dapp_xy * jy, d.p0, d.inv_p0);
-  qy = div_rcp(d.dapp_y * jy + d.dapp_yx * jx, d.p0, d.inv_p0);
+template <int N>
+__device__ __forceinline__ void detune_n(const phx_detuner &d, const P6 (&p)[N], double (&ux)[N],
+                                         double (&uy)[N]) {
+  if (d.type == PHX_DET_CHROMA) {
+    double ax[N], ay[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      ax[k] = d.cx[d.order - 1];
+      ay[k] = d.cy[d.order - 1];
+    }
+    for (int i = d.order - 2; i >= 0; --i)
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        ax[k] = fma(ax[k], p[k].dp, d.cx[i]);
+        ay[k] = fma(ay[k], p[k].dp, d.cy[i]);
+      }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      ux[k] = fma(ax[k], p[k].dp, ux[k]);
+      uy[k] = fma(ay[k], p[k].dp, uy[k]);
+    }
+  } else {
+    detune_amplitude_n<N>(d, p, ux, uy);
+  }
 }
 
 // The detuner sets with straight-line code (PHX_DETS_*): first-order
 // chromaticity (order-1 Horner: c0 * dp), then amplitude detuning; the
-// arithmetic of detune() for those sets.
-template <int DS>
-__device__ __forceinline__ void detune_set(const phx_tseg &t, const P6 &p, double &dx,
-                                           double &dy) {
-  dx = t.dQ_x;
-  dy = t.dQ_y;
+// arithmetic of detune_n for those sets.
+template <int N, int DS>
+__device__ __forceinline__ void detune_set_n(const phx_tseg &t, const P6 (&p)[N],
+                                             double (&ux)[N], double (&uy)[N]) {
   const phx_detuner &c = t.det[0];
-  dx = dx + c.cx[0] * p.dp;
-  dy = dy + c.cy[0] * p.dp;
-  if constexpr ((DS & ~PHX_DETS_SMOOTH) == PHX_DETS_C1_AMP) {
-    double qx, qy;
-    if constexpr ((DS & PHX_DETS_SMOOTH) != 0) detune_amplitude_smooth(t.det[1], p, qx, qy);
-    else detune_amplitude(t.det[1], p, qx, qy);
-    dx = dx + qx;
-    dy = dy + qy;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    ux[k] = fma(c.cx[0], p[k].dp, ux[k]);
+    uy[k] = fma(c.cy[0], p[k].dp, uy[k]);
   }
+  if constexpr ((DS & ~PHX_DETS_SMOOTH) == PHX_DETS_C1_AMP)
+    detune_amplitude_n<N, (DS & PHX_DETS_SMOOTH) != 0>(t.det[1], p, ux, uy);
 }
 
 // The element functions act on N particles at once: the element's constants
@@ -184,26 +222,18 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
       M22[k] = t.M22; M23[k] = t.M23; M32[k] = t.M32; M33[k] = t.M33;
     }
   } else {
-    double dphi_x[N], dphi_y[N];
+    // phases in turns, each detuner's shift added in order as the reference
+    // adds it
+    double u[2 * N], ux[N], uy[N], sn[2 * N], cs[2 * N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      ux[k] = t.dQ_x;
+      uy[k] = t.dQ_y;
+    }
     if constexpr (DS == PHX_DETS_GENERIC) {
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        dphi_x[k] = t.dQ_x;
-        dphi_y[k] = t.dQ_y;
-      }
-      for (int i = 0; i < nd; ++i) {
-        const phx_detuner &d = t.det[i];
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-          double qx, qy;
-          detune(d, p[k], qx, qy);
-          dphi_x[k] = dphi_x[k] + qx;
-          dphi_y[k] = dphi_y[k] + qy;
-        }
-      }
+      for (int i = 0; i < nd; ++i) detune_n<N>(t.det[i], p, ux, uy);
     } else {
-#pragma unroll
-      for (int k = 0; k < N; ++k) detune_set<DS>(t, p[k], dphi_x[k], dphi_y[k]);
+      detune_set_n<N, DS>(t, p, ux, uy);
     }
     const double I00 = t.I00, I01 = t.I01, I10 = t.I10, I11 = t.I11;
     const double I22 = t.I22, I23 = t.I23, I32 = t.I32, I33 = t.I33;
@@ -211,11 +241,13 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
     const double J22 = t.J22, J23 = t.J23, J32 = t.J32, J33 = t.J33;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      const double ax = dphi_x[k] * PHX_TWO_PI;
-      const double ay = dphi_y[k] * PHX_TWO_PI;
-      double sx, cx, sy, cy;
-      phx_sincos(ax, &sx, &cx);
-      phx_sincos(ay, &sy, &cy);
+      u[k] = ux[k];
+      u[N + k] = uy[k];
+    }
+    phx_sincos_turns_n<2 * N>(u, sn, cs);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const double sx = sn[k], cx = cs[k], sy = sn[N + k], cy = cs[N + k];
       if constexpr (SMOOTH) {
         // 1 * cos + 0 * sin and 0 * cos + J * sin, each rounded once: the
         // same values
@@ -229,14 +261,14 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
         M33[k] = cy;
         continue;
       }
-      M00[k] = I00 * cx + J00 * sx;
-      M01[k] = I01 * cx + J01 * sx;
-      M10[k] = I10 * cx + J10 * sx;
-      M11[k] = I11 * cx + J11 * sx;
-      M22[k] = I22 * cy + J22 * sy;
-      M23[k] = I23 * cy + J23 * sy;
-      M32[k] = I32 * cy + J32 * sy;
-      M33[k] = I33 * cy + J33 * sy;
+      M00[k] = fma(I00, cx, J00 * sx);
+      M01[k] = fma(J01, sx, I01 * cx);
+      M10[k] = fma(J10, sx, I10 * cx);
+      M11[k] = fma(I11, cx, J11 * sx);
+      M22[k] = fma(I22, cy, J22 * sy);
+      M23[k] = fma(J23, sy, I23 * cy);
+      M32[k] = fma(J32, sy, I32 * cy);
+      M33[k] = fma(I33, cy, J33 * sy);
     }
   }
   const bool disp = !SMOOTH && t.with_dispersion != 0;
@@ -249,10 +281,17 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
       q.y = q.y - dy0 * q.dp;
     }
     const double x = q.x, xp = q.xp, y = q.y, yp = q.yp;
-    q.x = M00[k] * x + M01[k] * xp;
-    q.xp = M10[k] * x + M11[k] * xp;
-    q.y = M22[k] * y + M23[k] * yp;
-    q.yp = M32[k] * y + M33[k] * yp;
+    if (nd == 0) {  // the reference's operations, bit for bit
+      q.x = M00[k] * x + M01[k] * xp;
+      q.xp = M10[k] * x + M11[k] * xp;
+      q.y = M22[k] * y + M23[k] * yp;
+      q.yp = M32[k] * y + M33[k] * yp;
+    } else {
+      q.x = fma(M00[k], x, M01[k] * xp);
+      q.xp = fma(M10[k], x, M11[k] * xp);
+      q.y = fma(M22[k], y, M23[k] * yp);
+      q.yp = fma(M32[k], y, M33[k] * yp);
+    }
     if (disp) {
       q.x = q.x + dx1 * q.dp;
       q.y = q.y + dy1 * q.dp;
@@ -265,55 +304,59 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
 // ---------------------------------------------------------------------------
 // STAT: a stationary RF sequence (PHX_SHAPE_STATIONARY): beta_ratio = 1,
 // phi_offset = phi_lock = p_increment = +0 and no dispersion, checked by the
-// host, so that 1 * z = z, (a + 0) + 0 = a + 0 and b - 0 = b drop those
-// terms with the same bits.
+// host, so that 1 * z = z, a phase offset of +0 and fma(dp, 1, -0) = dp drop
+// those terms with the same bits.
 template <int N, bool STAT = false>
 __device__ __forceinline__ void drift_n(P6 (&p)[N], const phx_long_op &o) {
   // Drift.track: z = beta_ratio*z - eta(dp)*dp*length   (:107-111)
-  const double eta0 = o.eta0, len = o.length;
+  const double e = -(o.eta0 * o.length);
   if constexpr (STAT) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) p[k].z = p[k].z - (eta0 * p[k].dp) * len;
+    for (int k = 0; k < N; ++k) p[k].z = fma(e, p[k].dp, p[k].z);
   } else {
     const double br = o.beta_ratio;
 #pragma unroll
-    for (int k = 0; k < N; ++k) p[k].z = br * p[k].z - (eta0 * p[k].dp) * len;
+    for (int k = 0; k < N; ++k) p[k].z = fma(e, p[k].dp, br * p[k].z);
   }
 }
 
 template <int N, bool STAT = false>
 __device__ __forceinline__ void rf_kick_n(P6 (&p)[N], const phx_long_op &o) {
-  // Kick.track_with_dispersion / track_without_dispersion (:185-203)
+  // Kick.track_with_dispersion / track_without_dispersion (:185-203):
+  //   phi = h (2 pi z / C) + phi_offset + phi_lock
+  //   dp = (dp p0_before + amplitude sin(phi) - p_increment) / p0_after
+  // with phi in turns and the quotients by C and p0_after folded into the
+  // kick's constants
+  const double hz = o.harmonic * o.inv_circumference, amp = o.amplitude * o.inv_p0_after;
+  double u[N], sn[N];
   if constexpr (STAT) {
-    const double h = o.harmonic, tp = o.two_pi, C = o.circumference;
-    const double p0b = o.p0_before, p0a = o.p0_after, amp = o.amplitude;
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-      P6 &q = p[k];
-      const double phi = h * div_rcp(tp * q.z, C, o.inv_circumference) + 0.0;
-      const double delta_p = q.dp * p0b;
-      q.dp = div_rcp(delta_p + amp * phx_sin(phi), p0a, o.inv_p0_after);
-    }
+    for (int k = 0; k < N; ++k) u[k] = fma(p[k].z, hz, 0.0);
+    phx_sin_turns_n<N>(u, sn);
+#pragma unroll
+    for (int k = 0; k < N; ++k) p[k].dp = fma(amp, sn[k], p[k].dp);
     return;
   }
   const bool disp = o.with_dispersion != 0;
-  const double Dx = o.D_x, Dy = o.D_y, h = o.harmonic, tp = o.two_pi, C = o.circumference;
-  const double off = o.phi_offset, lock = o.phi_lock, p0b = o.p0_before, p0a = o.p0_after;
-  const double amp = o.amplitude, pinc = o.p_increment;
+  const double Dx = o.D_x, Dy = o.D_y;
+  const double off = (o.phi_offset + o.phi_lock) * (1.0 / phx_math::TWO_PI);
+  const double ratio = o.p0_before == o.p0_after ? 1.0 : o.p0_before / o.p0_after;
+  const double pinc = -(o.p_increment * o.inv_p0_after);
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    P6 &q = p[k];
     if (disp) {
-      q.x = q.x - Dx * q.dp;
-      q.y = q.y - Dy * q.dp;
+      p[k].x = p[k].x - Dx * p[k].dp;
+      p[k].y = p[k].y - Dy * p[k].dp;
     }
-    const double phi = (h * div_rcp(tp * q.z, C, o.inv_circumference) + off) + lock;
-    double delta_p = q.dp * p0b;
-    delta_p = delta_p + (amp * phx_sin(phi) - pinc);
-    q.dp = div_rcp(delta_p, p0a, o.inv_p0_after);
+    u[k] = fma(p[k].z, hz, off);
+  }
+  phx_sin_turns_n<N>(u, sn);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    p[k].dp = fma(amp, sn[k], fma(p[k].dp, ratio, pinc));
     if (disp) {
-      q.x = q.x + Dx * q.dp;
-      q.y = q.y + Dy * q.dp;
+      p[k].x = p[k].x + Dx * p[k].dp;
+      p[k].y = p[k].y + Dy * p[k].dp;
     }
   }
 }
@@ -428,24 +471,28 @@ __device__ __forceinline__ void apply_shape_n(P6 (&p)[N], const phx_turn_program
 // z and dp after a program: only the longitudinal elements change them
 // (transverse segments act on x, xp, y, yp), so applying those alone gives
 // the same z and dp bit for bit.
-template <int SHAPE>
-__device__ __forceinline__ void apply_shape_longitudinal(P6 &q, const phx_turn_program &g) {
+template <int SHAPE, int N>
+__device__ __forceinline__ void apply_shape_longitudinal_n(P6 (&p)[N], const phx_turn_program &g) {
   constexpr int SH = SHAPE & ~PHX_SHAPE_STATIONARY;
   constexpr bool ST = SH != SHAPE;
-  P6(&p)[1] = *reinterpret_cast<P6(*)[1]>(&q);
   if constexpr (SH == PHX_SHAPE_RF1_T || SH == PHX_SHAPE_T_RF1) {
-    apply_rf_seq_n<1, 1, ST>(p, g.lseq[0]);
+    apply_rf_seq_n<1, N, ST>(p, g.lseq[0]);
   } else if constexpr (SH == PHX_SHAPE_RF2_T || SH == PHX_SHAPE_T_RF2) {
-    apply_rf_seq_n<2, 1, ST>(p, g.lseq[0]);
+    apply_rf_seq_n<2, N, ST>(p, g.lseq[0]);
   } else if constexpr (SH == PHX_SHAPE_LIN_T || SH == PHX_SHAPE_T_LIN) {
-    apply_linmap_n<1>(p, g.lin[0]);
+    apply_linmap_n<N>(p, g.lin[0]);
   } else if constexpr (SH == PHX_SHAPE_GENERIC) {
     for (int e = 0; e < g.n_el; ++e) {
       const int k = g.el_index[e];
-      if (g.el_type[e] == PHX_EL_LONG) apply_long_seq_n<1>(p, g.lseq[k]);
-      else if (g.el_type[e] == PHX_EL_LINMAP) apply_linmap_n<1>(p, g.lin[k]);
+      if (g.el_type[e] == PHX_EL_LONG) apply_long_seq_n<N>(p, g.lseq[k]);
+      else if (g.el_type[e] == PHX_EL_LINMAP) apply_linmap_n<N>(p, g.lin[k]);
     }
   }
+}
+
+template <int SHAPE>
+__device__ __forceinline__ void apply_shape_longitudinal(P6 &q, const phx_turn_program &g) {
+  apply_shape_longitudinal_n<SHAPE, 1>(*reinterpret_cast<P6(*)[1]>(&q), g);
 }
 
 __device__ __forceinline__ P6 (&one(P6 &p))[1] { return *reinterpret_cast<P6(*)[1]>(&p); }
@@ -501,15 +548,15 @@ __device__ __forceinline__ void apply_kick_set(P6 &p, int32_t idx, int n_slices,
 }
 
 // ---------------------------------------------------------------------------
-// Deterministic reductions.  Within a block: every thread stores its slot
-// values in LDS; for each slot, 16 threads each combine a fixed stride of
-// the PHX_BLOCK values (lanes q, q+16, q+32, ...), then one thread combines
-// the 16 results in order.  Across chunks: each thread folds a fixed stride
-// of chunks in increasing order, then the same block reduction.  For a given
-// particle count the association order is fixed, so results are
-// bit-reproducible, and a slot's result does not depend on which other
-// slots are reduced with it.  (An LDS transpose instead of wave shuffles:
-// the shuffle tree is a chain of dependent cross-lane permutes per slot.)
+// Deterministic reductions.  Within a block: each wave combines its 64 lanes
+// by data-parallel-primitive moves (row shifts by 1, 2, 4, 8, then the rows),
+// 18 vector instructions per slot and no barrier, and one thread per slot
+// then combines the waves in order.  (Through LDS, each slot's 256 values
+// read by 16 threads, took three barriers: 2.2 us of the 22 us pass at 1e6
+// macroparticles.)  Across chunks: each thread folds a fixed stride of chunks
+// in increasing order, then the same block reduction.  For a given particle
+// count the association order is fixed, so results are bit-reproducible, and
+// a slot's result does not depend on which other slots are reduced with it.
 // The operation of slot i is min if bit i of MINM is set, max if bit i of
 // MAXM is set, else sum.
 // ---------------------------------------------------------------------------
@@ -527,54 +574,62 @@ __device__ __forceinline__ double red_ident(int i) {
   return 0.0;
 }
 
-#define BR_GROUP 16  // slots per LDS round
-#define BR_PARTS 16  // partial results per slot
+// The value of v in the lane that the DPP control names, `old` where there is
+// none (a row's first lanes; rows outside ROWS).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double old, double v) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, ROWS,
+                                             0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, ROWS,
+                                             0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// Slot i's values of the wave's 64 lanes combined, in lane 63.
+template <unsigned long long MINM, unsigned long long MAXM>
+__device__ __forceinline__ double wave_reduce(int i, double v) {
+  const double id = red_ident<MINM, MAXM>(i);
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x111, 0xf>(id, v));  // row_shr:1
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x112, 0xf>(id, v));  // row_shr:2
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x114, 0xf>(id, v));  // row_shr:4
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x118, 0xf>(id, v));  // row_shr:8
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x142, 0xa>(id, v));  // row_bcast:15
+  v = red_slot<MINM, MAXM>(i, v, dpp_move<0x143, 0xc>(id, v));  // row_bcast:31
+  return v;
+}
 
 // LDS doubles needed by block_reduce_slots for NV slots.
-#define BR_LDS(NV) (((NV) < BR_GROUP ? (NV) : BR_GROUP) * (PHX_BLOCK + BR_PARTS))
+#define BR_LDS(NV) ((NV) * (PHX_BLOCK / PHX_WAVE))
 
-// Block-reduce NV slots held by the first PHX_BLOCK threads of the block
-// (every thread of the block must call it; larger blocks contribute only
-// their first PHX_BLOCK threads).  Thread t < NV gets the block result of
-// slot t as the return value (other threads: 0).  Slot t's operation is that
-// of bit OFF + t of the masks.  lds: __shared__ double[BR_LDS(NV)].
+// Block-reduce NV slots held by PHX_BLOCK threads of the block, t their index
+// among them (a block of several such groups reduces each in lds of its own;
+// every thread of the block calls it).  Thread t < NV gets the result of slot
+// t as the return value (other threads: 0).  Slot t's operation is that of bit
+// OFF + t of the masks.  lds: __shared__ double[BR_LDS(NV)].
+template <int NV, unsigned long long MINM, unsigned long long MAXM, int OFF = 0>
+__device__ __forceinline__ double block_reduce_slots_at(const double (&v)[NV], double *lds,
+                                                        const int t) {
+  constexpr int NW = PHX_BLOCK / PHX_WAVE;
+  static_assert(NV <= PHX_BLOCK, "one thread per slot");
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const double r = wave_reduce<MINM, MAXM>(OFF + i, v[i]);
+    if (t % PHX_WAVE == PHX_WAVE - 1) lds[(t / PHX_WAVE) * NV + i] = r;
+  }
+  lds_sync();
+  double out = 0.0;
+  if (t < NV) {
+    out = lds[t];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) out = red_slot<MINM, MAXM>(OFF + t, out, lds[w * NV + t]);
+  }
+  lds_sync();
+  return out;
+}
+
 template <int NV, unsigned long long MINM, unsigned long long MAXM, int OFF = 0>
 __device__ __forceinline__ double block_reduce_slots(const double (&v)[NV], double *lds) {
-  constexpr int G = NV < BR_GROUP ? NV : BR_GROUP;
-  constexpr int STRIDE = PHX_BLOCK / BR_PARTS;
-  double *part = lds + G * PHX_BLOCK;
-  const int t = threadIdx.x;
-  double out = 0.0;
-#pragma unroll
-  for (int g0 = 0; g0 < NV; g0 += G) {
-    if (t < PHX_BLOCK) {
-#pragma unroll
-      for (int i = 0; i < G; ++i)
-        if (g0 + i < NV) lds[i * PHX_BLOCK + t] = v[g0 + i];
-    }
-    lds_sync();
-    if (t < G * BR_PARTS) {
-      const int i = t / BR_PARTS, q = t % BR_PARTS;
-      if (g0 + i < NV) {
-        const int k = OFF + g0 + i;
-        const double *row = lds + i * PHX_BLOCK;
-        double r = row[q];
-#pragma unroll
-        for (int m = 1; m < STRIDE; ++m) r = red_slot<MINM, MAXM>(k, r, row[m * BR_PARTS + q]);
-        part[i * BR_PARTS + q] = r;
-      }
-    }
-    lds_sync();
-    if (t >= g0 && t < g0 + G && t < NV) {
-      const int i = t - g0, k = OFF + t;
-      double r = part[i * BR_PARTS];
-#pragma unroll
-      for (int q = 1; q < BR_PARTS; ++q) r = red_slot<MINM, MAXM>(k, r, part[i * BR_PARTS + q]);
-      out = r;
-    }
-    lds_sync();
-  }
-  return out;
+  return block_reduce_slots_at<NV, MINM, MAXM, OFF>(v, lds, threadIdx.x);
 }
 
 // Reduce per-chunk partials part[c*NV + i] over c < n_chunks into res[i]
@@ -587,13 +642,15 @@ __device__ __forceinline__ double block_reduce_slots(const double (&v)[NV], doub
 // same value).  The order depends on nc only, not on the block size, so
 // every fold of the same partials gives the same bits.  The waves of the
 // block take slots i0 + w, i0 + w + W, ...; res[i] receives slot i.  Ends
-// with a barrier.
-template <unsigned long long MINM, unsigned long long MAXM>
+// with a barrier.  SKIP >= 0: slot SKIP - 1 is left out (the next slot takes
+// its place, so i1 - i0 slots are folded).
+template <unsigned long long MINM, unsigned long long MAXM, int SKIP = -1>
 __device__ __forceinline__ void fold_partials(const double *part, int64_t nc, int i0, int i1,
                                               double *res) {
   const int lane = threadIdx.x % PHX_WAVE, wv = threadIdx.x / PHX_WAVE;
   const int nw = blockDim.x / PHX_WAVE;
-  for (int i = i0 + wv; i < i1; i += nw) {
+  for (int q = i0 + wv; q < i1; q += nw) {
+    const int i = SKIP >= 0 && q >= SKIP - 1 ? q + 1 : q;
     const double *row = part + (size_t)i * nc;
     const double id = red_ident<MINM, MAXM>(i);
     double acc = id;
@@ -619,30 +676,65 @@ __device__ __forceinline__ void fold_partials(const double *part, int64_t nc, in
 }
 
 // ---------------------------------------------------------------------------
-// Split 64-bit fixed-point accumulation of per-slice sums.
-// A value u with |u| <= B is scaled by 2^e, e = 60 - ilogb(B), so
-// |q| = |rint(u*2^e)| < 2^61; q = hi*2^32 + lo with lo in [0, 2^32).
-// Sums of hi (int64) and lo (uint64) are exact for up to 2^31 particles per
-// slice, so the per-slice sum is independent of summation order.
+// Fixed-point accumulation of per-slice sums, in two 64-bit limbs.
+// With |u| <= lim = 2^P and s = 2^(FX_HB - P): u s = h + r, h = rint(u s)
+// (|h| <= 2^FX_HB), and l = rint(r 2^FX_LB), so u is kept to an absolute
+// 2^(P - FX_HB - FX_LB) (2^-64 lim or finer for any bound the scale was taken
+// from) and its sums are integer sums, independent of the order.
+// Both limbs come from one FMA with the constant FX_MAGIC = 1.5 * 2^52, whose
+// unit in the last place is 1: t = fma(u, s, FX_MAGIC) rounds u s to an
+// integer that stands in t's low mantissa bits, so the 64-bit patterns of t
+// are summed as they are (modulo 2^64) and bits(FX_MAGIC) times the number of
+// terms is subtracted once per slice (acc_lds_store).  A value costs four
+// FP64 operations (fma, subtract, fma, fma) where ldexp, llrint and 64-bit
+// shifts and masks took about twenty instructions.
+// The scale's P is rounded up to a multiple of 8 above twice the bound: the
+// scale of a state and that of the turn before it (the fused engine's) agree
+// unless the bound crosses such a power of two.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int fx_exponent(double bound) {
-  if (!(bound > 0.0) || !isfinite(bound)) return 0;
-  return 60 - ilogb(bound);
+#define FX_LB 40
+#define FX_HB 33
+#define FX_MAGIC 6755399441055744.0  // 1.5 * 2^52
+#define FX_MAGIC_BITS 0x4338000000000000ULL
+#define FX_HUGE 0x1p1000  // beyond (and NaN): summed in FP64 as it is
+
+struct FxScale {
+  double s, lim, unit;  // 2^(hb - P), 2^P, and the value of h = 1: 2^(P - hb)
+};
+
+// 2^k, |k| <= 1022
+__device__ __forceinline__ double fx_pow2(int k) {
+  return __longlong_as_double((long long)(1023 + k) << 52);
 }
 
-__device__ __forceinline__ void fx_split(double u, int e, unsigned long long &hi,
-                                         unsigned long long &lo) {
-  const long long q = llrint(ldexp(u, e));
-  hi = (unsigned long long)(q >> 32);
-  lo = (unsigned long long)(q & 0xffffffffLL);
+// n: the largest number of terms of a sum; its h limb stays below 2^62 (FX_HB
+// bits for up to 2^29 terms).
+__device__ __forceinline__ FxScale fx_scale(double bound, int64_t n) {
+  int P = 0;
+  if (bound > 0.0 && bound < FX_HUGE) {
+    // frexp's exponent is ilogb + 1; rounded up to a multiple of 8
+    P = (__builtin_amdgcn_frexp_exp(bound) + 1 + 7) & ~7;
+    P = P < -944 ? -944 : P;
+  }
+  int hb = FX_HB;
+  if (n >> 29) hb -= 64 - __clzll((unsigned long long)(n >> 29));
+  return FxScale{fx_pow2(hb - P), fx_pow2(P), fx_pow2(P - hb)};
 }
 
+// Sum of the limbs and of the out-of-range parts `over` (fallback sums:
+// multiples of lim, exact in FP64, unless a term was not finite), as a
+// correctly rounded double.
 __device__ __forceinline__ double fx_value(unsigned long long hi_sum, unsigned long long lo_sum,
-                                           int e) {
-  const long long h = (long long)hi_sum + (long long)(lo_sum >> 32);
-  const double top = ldexp((double)h, 32);
-  const double s = top + (double)(lo_sum & 0xffffffffULL);
-  return ldexp(s, -e);
+                                           double over, const FxScale &f) {
+  long long h = (long long)hi_sum + ((long long)lo_sum >> FX_LB);
+  const double oh = over * f.s;  // in units of h
+  const bool in = fabs(oh) < 0x1p61;
+  if (in) h += (long long)oh;
+  const double a = (double)h;  // |h| may exceed 53 bits: keep the remainder
+  const long long r = h - (long long)a;
+  const double b = (double)(r * (1LL << FX_LB) + (long long)(lo_sum & ((1ULL << FX_LB) - 1ULL)));
+  const double v = fma(b, 1.0 / (double)(1LL << FX_LB), a) * f.unit;
+  return in ? v : v + over;
 }
 
 // ---------------------------------------------------------------------------

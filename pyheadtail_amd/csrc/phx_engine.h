@@ -28,9 +28,21 @@ namespace phx_en {
 
 inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
+// What a pass that slices its own turn (ahead_body) needs before it starts,
+// formed by the merge of the turn before it: the turn's cuts, the bounds of
+// x and y that scale its fixed-point sums (those of the state before it),
+// the shift of its z sums (particle 0's z one turn on) and the wake ring's
+// slot and filling after the turn.  One per parity of the turn.
+struct AheadState {
+  double tail, head, width, mean_z, sigma_z, absx, absy, zshift;
+  int nh, nf;
+};
+
 struct EngineWs {
   double *partials;   // [EN_NV][pass grid] (slot-major)
   double *p0;         // particle 0 before the pass: the shifts of its sums
+  AheadState *ahead;  // [2] (turn parity), in the rest of p0's 256 bytes
+  int *cur_turn;      // the turn of the last such pass
   AccParts acc;       // H partial histograms, T = 2 (x, y)
   double *conv_part;  // [n_kicks][conv_rows(S, T)][S]
 };
@@ -50,6 +62,9 @@ __host__ __device__ inline EngineWs engine_ws(void *ws, int64_t n, int S) {
   w.partials = reinterpret_cast<double *>(p);
   p += ((size_t)nc * EN_NV * 8 + 255) / 256 * 256;
   w.p0 = reinterpret_cast<double *>(p);
+  w.ahead = reinterpret_cast<AheadState *>(p + 64);
+  w.cur_turn = reinterpret_cast<int *>(p + 64 + 2 * sizeof(AheadState));
+  static_assert(64 + 2 * sizeof(AheadState) + sizeof(int) <= 256, "p0 region");
   p += 256;
   const int H = hist_blocks(n);
   w.acc = acc_parts_layout(p, H, Se, 2);
@@ -87,6 +102,9 @@ struct EngineArgs {
   int T;
   int grid;  // blocks of the particle pass (its partials: [slot][grid])
   int gmax;  // kicks one convolution block serves (LDS permitting)
+  int nsub;  // three-launch turns: groups of PHX_BLOCK threads per pass block
+             // (0: they do not apply)
+  int hblk;  // and the pass's blocks, each storing one partial histogram
 };
 
 // ---------------------------------------------------------------------------
@@ -135,8 +153,7 @@ inline size_t sc_ws_bytes(int64_t n, int S) {
 struct ScCtx {
   const ScSlice *sl;
   const WofzCoeffs *wc;
-  double tail, width, inv_width;
-  int S;
+  SliceBins bins;
 };
 
 template <int N>
@@ -146,9 +163,9 @@ __device__ __forceinline__ void sc_kick_n(P6 (&p)[N], const ScCtx &c, const phx_
   bool in[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    const double fl = slice_floor_r(p[k].z, c.tail, c.width, c.inv_width);
-    in[k] = fl >= 0.0 && fl < (double)c.S;
-    const ScSlice &q = c.sl[in[k] ? (int)fl : 0];
+    const int s = c.bins.index(p[k].z);
+    in[k] = s >= 0;
+    const ScSlice &q = c.sl[in[k] ? s : 0];
     dx[k] = p[k].x - q.mx;
     dy[k] = p[k].y - q.my;
     nl[k] = q.nl;
@@ -187,10 +204,9 @@ __device__ __forceinline__ void store_p(const phx_engine &e, int64_t j, const P6
 // nk = min(program kicks, engine kicks): the kick table holds the latter.
 template <int KS>
 __device__ __forceinline__ void kick_pending(P6 &p, const phx_turn_program &g, int nk,
-                                             double tail, double width, double inv_width,
-                                             int S, const double *kicks) {
-  const double f = slice_floor_r(p.z, tail, width, inv_width);
-  if (f >= 0.0 && f < (double)S) apply_kick_set<KS>(p, (int32_t)f, S, g.kick, nk, kicks);
+                                             const SliceBins &bins, int S, const double *kicks) {
+  const int s = bins.index(p.z);
+  if (s >= 0) apply_kick_set<KS>(p, s, S, g.kick, nk, kicks);
 }
 
 // The pending kick's table values for the PHX_PPT particles of a group,
@@ -206,13 +222,13 @@ struct KickAhead {
   static constexpr bool ON = NV > 0;
   double k[PHX_PPT][NV > 0 ? NV : 1];
   bool in[PHX_PPT];
-  __device__ __forceinline__ void fetch(const P6 (&q)[PHX_PPT], double tail, double width,
-                                        double inv_width, int S, const double *kicks) {
+  __device__ __forceinline__ void fetch(const P6 (&q)[PHX_PPT], const SliceBins &bins, int S,
+                                        const double *kicks) {
 #pragma unroll
     for (int j = 0; j < PHX_PPT; ++j) {
-      const double f = slice_floor_r(q[j].z, tail, width, inv_width);
-      in[j] = f >= 0.0 && f < (double)S;
-      const int s = in[j] ? (int)f : 0;  // slot 0 is read and not used outside
+      const int b = bins.index(q[j].z);
+      in[j] = b >= 0;
+      const int s = in[j] ? b : 0;  // slot 0 is read and not used outside
 #pragma unroll
       for (int i = 0; i < NV; ++i) k[j][i] = kicks[(size_t)i * S + s];
     }
@@ -283,14 +299,14 @@ __device__ __forceinline__ double *at_off(double *b, uint32_t off) {
   return reinterpret_cast<double *>(reinterpret_cast<char *>(b) + off);
 }
 
-// The PHX_PPT particles of this thread in the group starting at byte offset
+// The PHX_PPT particles of thread tid in the group starting at byte offset
 // goff; lim: the group's particle count if it is the partial last group,
 // else PHX_CHUNK (no guard needed).
-__device__ __forceinline__ void group_load(const GroupPtr &gb, uint32_t goff, int lim,
+__device__ __forceinline__ void group_load(const GroupPtr &gb, uint32_t goff, int lim, int tid,
                                            P6 (&p)[PHX_PPT]) {
 #pragma unroll
   for (int k = 0; k < PHX_PPT; ++k) {
-    const int o = (int)threadIdx.x + k * PHX_BLOCK;
+    const int o = tid + k * PHX_BLOCK;
     const uint32_t off = goff + (uint32_t)o * 8u;
     if (lim == PHX_CHUNK || o < lim)
       p[k] = P6{ld_pos(at_off(gb.c[0], off)), ld_mom(at_off(gb.c[1], off)),
@@ -301,11 +317,11 @@ __device__ __forceinline__ void group_load(const GroupPtr &gb, uint32_t goff, in
   }
 }
 
-__device__ __forceinline__ void group_store(const GroupPtr &gb, uint32_t goff, int lim,
+__device__ __forceinline__ void group_store(const GroupPtr &gb, uint32_t goff, int lim, int tid,
                                             const P6 (&p)[PHX_PPT]) {
 #pragma unroll
   for (int k = 0; k < PHX_PPT; ++k) {
-    const int o = (int)threadIdx.x + k * PHX_BLOCK;
+    const int o = tid + k * PHX_BLOCK;
     const uint32_t off = goff + (uint32_t)o * 8u;
     if (lim == PHX_CHUNK || o < lim) {
       *at_off(gb.c[0], off) = p[k].x; st_mom(at_off(gb.c[1], off), p[k].xp);
@@ -363,26 +379,54 @@ struct PassLayout {
 // turn (stage: the offset of the stage's program from the turn's first;
 // the later stages run sc_pass_body).  The pending wake kick and the
 // statistics belong to stage 0.
-template <int MODE, bool REC, bool WAKE, int SHAPE, int KS, int DS>
+// AHEAD: one of ahead_body's groups of threads (tid: the thread's index in
+// it, lds its reduction area): the turn's cuts are known, the moved particles
+// are added to the block's slice histogram `acc`, and the z sums are those of
+// the next turn (aheadz: the cuts and scales of ahead_body; bid >= nblk: a
+// group without particles).
+struct AheadCtx {
+  AccLds acc;
+  const double *kicks;  // the pending kick table in LDS
+  SliceBins bins;
+  FxScale fx, fy;
+};
+
+// The dipole or plates kick of one particle of slice s (>= 0) from the table
+// in LDS, with apply_kick_set's operations.
+template <int KS>
+__device__ __forceinline__ void kick_from_lds(P6 &p, int s, int S, const double *kicks) {
+  p.xp = p.xp + kicks[s];
+  if constexpr (KS == PHX_KICKS_DXDY) {
+    p.yp = p.yp + kicks[S + s];
+  } else {
+    p.xp = p.xp + kicks[S + s] * p.x;
+    p.yp = p.yp + kicks[2 * S + s];
+    p.yp = p.yp + kicks[3 * S + s] * p.y;
+  }
+}
+
+template <int MODE, bool REC, bool WAKE, int SHAPE, int KS, int DS, bool AHEAD>
 __device__ __forceinline__ void pass_body(
     const EngineArgs &a, double *__restrict__ x, double *__restrict__ xp,
     double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
     double *__restrict__ dp, const phx_turn_program *__restrict__ programs,
-    const double *__restrict__ kicks, int bid, int nblk, int stage = 0) {
+    const double *__restrict__ kicks, int bid, int nblk, int stage, int tid, double *lds,
+    const AheadCtx *ctx) {
   using L = PassLayout<REC, WAKE>;
+  static_assert(!AHEAD || (MODE == 0 && WAKE && KS != PHX_KICKS_GENERIC), "ahead pass");
   const phx_engine &e = a.e;
-  extern __shared__ double pass_lds[];
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
   const int64_t n = e.n;
   const int turn = *e.turn_counter;
   const int prog_turn = MODE == 0 ? turn : (turn > 0 ? turn - 1 : 0);
   const phx_turn_program &g = programs[e.turn_program[prog_turn] + stage];
   const int pend = stage == 0 ? *e.pending : 0;
-  const double tail = e.state->tail, width = e.state->width;
-  const double inv_width = 1.0 / width;
   const int S = e.n_slices;
+  const SliceBins bins(e.state->tail, e.state->width, S);
+  // the cuts after this pass: a space-charge slicing's, or the wake's
+  const bool minmax = (g.has_sc ? g.sc_slicer : g.slicer).cuts_mode == PHX_CUTS_MINMAX;
   const int nk = g.n_kicks < a.n_kicks ? g.n_kicks : a.n_kicks;
-  const int64_t ng = phx_n_groups(n);
+  const int64_t ng = AHEAD && bid >= nblk ? 0 : phx_n_groups(n);
   // the group's base pointers and particle count (uniform)
   const GroupPtr gb{{x, xp, y, yp, z, dp}};
   // the group's byte offset and particle count (uniform)
@@ -393,59 +437,75 @@ __device__ __forceinline__ void pass_body(
     return rest >= PHX_CHUNK ? PHX_CHUNK : (int)rest;
   };
   int64_t gi = bid;
-  uint32_t gc, gnx = 0;
-  int lc = group(gi, gc);
+  uint32_t gc = 0, gnx = 0;
+  int lc = 0;
+  if (!AHEAD || gi < ng) lc = group(gi, gc);
   P6 cur[PHX_PPT], nxt[PHX_PPT];
-  group_load(gb, gc, lc, cur);
+  group_load(gb, gc, lc, tid, cur);
   // Particle 0 sets the shifts of the shifted sums (stats.pyx:cov): its
   // state after the pending kick (statistics), and its z after this turn's
   // elements (cuts), which needs the kick only where a kick changes dp and
   // only the longitudinal elements.  Every lane computes it (uniform values;
   // once per block) from the snapshot taken before this pass: block 0
-  // rewrites particle 0 while later blocks may still be starting.
+  // rewrites particle 0 while later blocks may still be starting.  (AHEAD:
+  // the merge of the turn before left the z shift in the workspace.)
   double src[7];
-  {
+  if constexpr (!AHEAD || REC) {
     const double *p0 = w.p0;
     P6 q = P6{p0[0], p0[1], p0[2], p0[3], p0[4], p0[5]};
     bool kick_dp = false;
     if constexpr (KS == PHX_KICKS_GENERIC) {
       for (int k = 0; k < nk; ++k) kick_dp = kick_dp || g.kick[k].plane == PHX_PLANE_DP;
     }
-    if (pend && (REC || kick_dp)) kick_pending<KS>(q, g, nk, tail, width, inv_width, S, kicks);
+    if constexpr (AHEAD) {
+      const int b = bins.index(q.z);
+      if (pend && b >= 0) kick_from_lds<KS>(q, b, S, ctx->kicks);
+    } else {
+      if (pend && (REC || kick_dp)) kick_pending<KS>(q, g, nk, bins, S, kicks);
+    }
     src[0] = q.x; src[1] = q.xp; src[2] = q.y; src[3] = q.yp; src[4] = q.z; src[5] = q.dp;
-    if (MODE == 0) apply_shape_longitudinal<SHAPE>(q, g);
+    if (MODE == 0 && !AHEAD) apply_shape_longitudinal<SHAPE>(q, g);
     src[6] = q.z;
   }
+  if constexpr (AHEAD) src[6] = w.ahead[turn & 1].zshift;
   double v[L::NV];
 #pragma unroll
   for (int i = 0; i < L::NV; ++i) v[i] = red_ident<L::MINM, L::MAXM>(i);
   double shs[6];
 #pragma unroll
-  for (int i = 0; i < 6; ++i) shs[i] = src[i];
+  for (int i = 0; i < 6; ++i) shs[i] = AHEAD && !REC ? 0.0 : src[i];
   const double zshift = src[6];
+  // four-launch pass: the kick's table values are read one group ahead
+  constexpr bool KA = KickAhead<KS>::ON && !AHEAD;
   KickAhead<KS> ka;
-  if (KickAhead<KS>::ON && pend) ka.fetch(cur, tail, width, inv_width, S, kicks);
+  if (KA && pend) ka.fetch(cur, bins, S, kicks);
   for (; gi < ng; gi += nblk) {
     const int64_t gn = gi + nblk;
     int ln = 0;
     if (gn < ng) {
       ln = group(gn, gnx);
-      group_load(gb, gnx, ln, nxt);
+      group_load(gb, gnx, ln, tid, nxt);
     }
     if (pend) {
-      if constexpr (KickAhead<KS>::ON) {
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int k = 0; k < PHX_PPT; ++k) {
+          const int b = bins.index(cur[k].z);
+          if (b >= 0) kick_from_lds<KS>(cur[k], b, S, ctx->kicks);
+        }
+      } else if constexpr (KA) {
         ka.apply(cur);
       } else {
 #pragma unroll
         for (int k = 0; k < PHX_PPT; ++k)
-          kick_pending<KS>(cur[k], g, nk, tail, width, inv_width, S, kicks);
+          kick_pending<KS>(cur[k], g, nk, bins, S, kicks);
       }
     }
     const bool full = lc == PHX_CHUNK;
     if (REC) {
 #pragma unroll
       for (int k = 0; k < PHX_PPT; ++k)
-        if (full || (int)threadIdx.x + k * PHX_BLOCK < lc)
+        if (full || tid + k * PHX_BLOCK < lc)
           stats_accumulate(&v[L::SOFF], cur[k], shs);
     }
     if (MODE == 0) {
@@ -459,29 +519,247 @@ __device__ __forceinline__ void pass_body(
 #endif
       apply_shape_n<SHAPE, PHX_PPT, DS>(cur, *gl);
     }
+    if (MODE == 0 || pend) group_store(gb, gc, lc, tid, cur);
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int k = 0; k < PHX_PPT; ++k) {
+        if (full || tid + k * PHX_BLOCK < lc) {
+          const int s = ctx->bins.index(cur[k].z);
+          if (s >= 0) {
+            atomicAdd(&ctx->acc.counts[s], 1u);
+            acc_add_value(ctx->acc, S, 0, s, cur[k].x, ctx->fx, w.acc.fallback);
+            acc_add_value(ctx->acc, S, 1, s, cur[k].y, ctx->fy, w.acc.fallback);
+          }
+        }
+      }
+      apply_shape_longitudinal_n<SHAPE, PHX_PPT>(cur, g);  // z one turn on
+    }
     if (WAKE) {
 #pragma unroll
       for (int k = 0; k < PHX_PPT; ++k) {
-        if (full || (int)threadIdx.x + k * PHX_BLOCK < lc) {
+        if (full || tid + k * PHX_BLOCK < lc) {
           double zb[ZB_NV];
 #pragma unroll
           for (int i = 0; i < ZB_NV; ++i) zb[i] = v[i];
-          zblock_accumulate<0x05u>(zb, cur[k], zshift);  // max |x|, |y|: the histogram's
+          // max |x|, |y| only scale the slices' fixed-point sums, which take
+          // larger values too (acc_add_value): every PHX_PPT-th particle's do
+          if (k == 0) zblock_accumulate<0x05u>(zb, cur[k], zshift, minmax);
+          else zblock_accumulate<0u>(zb, cur[k], zshift, minmax);
 #pragma unroll
           for (int i = 0; i < ZB_NV; ++i) v[i] = zb[i];
         }
       }
     }
-    if (MODE == 0 || pend) group_store(gb, gc, lc, cur);
 #pragma unroll
     for (int k = 0; k < PHX_PPT; ++k) cur[k] = nxt[k];
     gc = gnx;
     lc = ln;
     // the next group's kick values, while this block's other waves compute
-    if (KickAhead<KS>::ON && pend && gn < ng) ka.fetch(cur, tail, width, inv_width, S, kicks);
+    if (KA && pend && gn < ng) ka.fetch(cur, bins, S, kicks);
   }
-  const double r = block_reduce_slots<L::NV, L::MINM, L::MAXM>(v, pass_lds);
-  if (threadIdx.x < L::NV) w.partials[(size_t)threadIdx.x * nblk + bid] = r;
+  if constexpr (AHEAD) {
+    // the z sums and the maxima of |x| and |y| (the other slots are not kept)
+    double c[ZA_NV];
+#pragma unroll
+    for (int i = 0; i < ZA_NV; ++i) c[i] = v[za_slot(i)];
+    const double r = block_reduce_slots_at<ZA_NV, ZA_MINM, ZA_MAXM>(c, lds, tid);
+    if (bid < nblk && tid < ZA_NV) w.partials[(size_t)za_slot(tid) * nblk + bid] = r;
+    if constexpr (REC) {
+      double t[EN_STAT_NV];
+#pragma unroll
+      for (int i = 0; i < EN_STAT_NV; ++i) t[i] = v[L::SOFF + i];
+      const double q = block_reduce_slots_at<EN_STAT_NV, 0ULL, 0ULL>(t, lds, tid);
+      if (bid < nblk && tid < EN_STAT_NV) w.partials[(size_t)(L::SOFF + tid) * nblk + bid] = q;
+    }
+  } else {
+    const double r = block_reduce_slots<L::NV, L::MINM, L::MAXM>(v, lds);
+    if (threadIdx.x < L::NV) w.partials[(size_t)threadIdx.x * nblk + bid] = r;
+  }
+}
+
+template <int MODE, bool REC, bool WAKE, int SHAPE, int KS, int DS>
+__device__ __forceinline__ void pass_body(
+    const EngineArgs &a, double *__restrict__ x, double *__restrict__ xp,
+    double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
+    double *__restrict__ dp, const phx_turn_program *__restrict__ programs,
+    const double *__restrict__ kicks, int bid, int nblk, int stage = 0) {
+  extern __shared__ double pass_lds[];
+  pass_body<MODE, REC, WAKE, SHAPE, KS, DS, false>(a, x, xp, y, yp, z, dp, programs, kicks, bid,
+                                                   nblk, stage, threadIdx.x, pass_lds, nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// Three-launch turns (EngineArgs.nsub > 0): pass with slicing, merge,
+// convolution.  The cuts of a turn depend on z after its elements, which the
+// longitudinal motion alone fixes (no kick on dp), so the pass of turn t can
+// also sum z of turn t + 1 (the same program every turn) from the particles
+// it holds: the merge folds those sums into the cuts of turn t + 1, and the
+// pass of turn t + 1 slices each particle as it moves it.  The slice
+// histogram's own launch and its 24 B per macroparticle go (11.2 of 45.4 us
+// at 1e6 macroparticles, 42.6 of 231 us at 1e7), for a second evaluation of
+// the longitudinal motion (nothing for a linear map, a sine for an RF kick).
+// One pass block is nsub groups of PHX_BLOCK threads, each a block of the
+// four-launch pass (the same particles in the same order, hence the same z
+// sums, cuts and coordinates bit for bit), sharing one histogram: a CU then
+// stores one partial histogram, as many as the histogram kernel stored.
+// ---------------------------------------------------------------------------
+__host__ __device__ inline size_t ahead_hist_doubles(int S) {
+  return (acc_lds_bytes(S, 2) + 7) / 8;
+}
+// and the pending kick's table, which every particle reads at its slice: from
+// global memory, 2 or 4 gathers per particle of a table that the streamed
+// coordinates push out of the L1 (26.6 us against 20 us for a linear-map pass
+// with a 1000-slice plates kick)
+__host__ __device__ inline size_t ahead_kick_doubles(int S, int kick_shape) {
+  return (size_t)(kick_shape == PHX_KICKS_PLATES ? 4 : 2) * S;
+}
+// LDS doubles of one group's reduction
+template <bool REC>
+__host__ __device__ constexpr int ahead_red_doubles() {
+  return REC ? BR_LDS(EN_STAT_NV) : BR_LDS(ZA_NV);
+}
+// Groups of threads per block: three of the specialised passes' groups fill a
+// CU (at most 168 vector registers), two of the others'.
+template <bool REC, int SHAPE>
+constexpr int ahead_nsub() {
+  return REC || SHAPE == PHX_SHAPE_GENERIC ? 2 : 3;
+}
+
+// The partial histograms of a three-launch turn: hblk of them, the fallback
+// sums where the four-launch turn has them.
+__device__ __forceinline__ AccParts ahead_parts(const EngineWs &w, int S, int hblk) {
+  AccParts P = acc_parts_layout(w.acc.cnt, hblk, S, 2);
+  P.fallback = w.acc.fallback;
+  return P;
+}
+
+// Pass block kb of nkb.
+template <bool REC, int SHAPE, int KS, int DS>
+__device__ __forceinline__ void ahead_body(
+    const EngineArgs &a, double *__restrict__ x, double *__restrict__ xp,
+    double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
+    double *__restrict__ dp, const phx_turn_program *__restrict__ programs,
+    const double *__restrict__ kicks, int kb, int nkb, int nsub) {
+  extern __shared__ double pass_lds[];
+  const phx_engine &e = a.e;
+  const int S = e.n_slices;
+  const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x / PHX_BLOCK);
+  const int tid = threadIdx.x % PHX_BLOCK;
+  double *kt = pass_lds + ahead_hist_doubles(S);
+  double *red = kt + ahead_kick_doubles(S, KS) + sub * ahead_red_doubles<REC>();
+  EngineWs w = engine_ws(e.ws, e.n, S);
+  AheadCtx c;
+  c.kicks = kt;
+  c.acc = acc_lds_layout(reinterpret_cast<unsigned long long *>(pass_lds), S, 2);
+  for (int i = threadIdx.x; i < (int)ahead_kick_doubles(S, KS); i += blockDim.x) kt[i] = kicks[i];
+  acc_lds_zero(c.acc, S, 2);  // ends with a barrier; the particle loads follow it
+  const int turn = *e.turn_counter;
+  const AheadState &h = w.ahead[turn & 1];
+  c.bins = SliceBins(h.tail, h.width, S);
+  c.fx = fx_scale(h.absx, e.n);
+  c.fy = fx_scale(h.absy, e.n);
+  for (int b0 = 0; b0 < a.grid; b0 += nkb * nsub)
+    pass_body<0, REC, true, SHAPE, KS, DS, true>(a, x, xp, y, yp, z, dp, programs, kicks,
+                                                 b0 + sub * nkb + kb, a.grid, 0, tid, red, &c);
+  if (kb == 0 && threadIdx.x == 0) *w.cur_turn = turn;
+  acc_lds_store(c.acc, S, 2, ahead_parts(w, S, a.hblk), kb);
+}
+
+// The cuts of a three-launch turn from folded z sums, the bounds of |x| and
+// |y| and the ring's state after that turn, into its AheadState (one thread).
+__device__ __forceinline__ void ahead_set(AheadState &h, const phx_slicer &cfg, int64_t n,
+                                          const double *res, int nh, int nf) {
+  phx_slice_state st;
+  compute_cuts(cfg, n, res[0], res[1], res[2], res[3], res[4], st);
+  h.tail = st.tail;
+  h.head = st.head;
+  h.width = st.width;
+  h.mean_z = st.mean_z;
+  h.sigma_z = st.sigma_z;
+  h.absx = res[5];
+  h.absy = res[7];
+  h.nh = nh;
+  h.nf = nf;
+}
+
+// Particle 0's z after two turns' longitudinal motion from c: the shift of
+// the z sums that the next pass forms.
+__device__ __forceinline__ double ahead_shift(double *const *c, const phx_turn_program &g) {
+  P6 q = P6{0.0, 0.0, 0.0, 0.0, c[4][0], c[5][0]};
+  apply_shape_longitudinal<PHX_SHAPE_GENERIC>(q, g);
+  apply_shape_longitudinal<PHX_SHAPE_GENERIC>(q, g);
+  return q.z;
+}
+
+__device__ __forceinline__ void ahead_fold(const double *partials, int grid, double *res) {
+  fold_partials<ZB_MINM, ZB_MAXM, ZA_NV>(partials, grid, 0, ZA_NV, res);
+}
+
+// Before the first three-launch turn of a sequence: block bid of grid sums
+// the z that the next turn's longitudinal motion gives the current state, in
+// the pass's order, and the maxima of |x| and |y|; ahead_start_fold (one
+// block) then sets the turn's AheadState.
+__device__ __forceinline__ void ahead_start_body(const EngineArgs &a, int bid) {
+  const phx_engine &e = a.e;
+  extern __shared__ double pass_lds[];
+  EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
+  const int turn = *e.turn_counter;
+  const phx_turn_program &g = e.programs[e.turn_program[turn]];
+  double *const *c = e.coords;
+  const bool minmax = g.slicer.cuts_mode == PHX_CUTS_MINMAX;
+  double zshift;
+  {
+    P6 q = P6{0.0, 0.0, 0.0, 0.0, c[4][0], c[5][0]};
+    apply_shape_longitudinal<PHX_SHAPE_GENERIC>(q, g);
+    zshift = q.z;
+  }
+  double v[ZB_NV];
+#pragma unroll
+  for (int i = 0; i < ZB_NV; ++i) v[i] = red_ident<ZB_MINM, ZB_MAXM>(i);
+  const int64_t ng = phx_n_groups(e.n);
+  for (int64_t gi = bid; gi < ng; gi += a.grid) {
+    P6 p[PHX_PPT];
+#pragma unroll
+    for (int k = 0; k < PHX_PPT; ++k) {
+      const int64_t j = gi * PHX_CHUNK + threadIdx.x + k * PHX_BLOCK;
+      p[k] = P6{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      if (j < e.n) {
+        p[k].x = c[0][j];
+        p[k].y = c[2][j];
+        p[k].z = c[4][j];
+        p[k].dp = c[5][j];
+      }
+    }
+    apply_shape_longitudinal_n<PHX_SHAPE_GENERIC, PHX_PPT>(p, g);
+#pragma unroll
+    for (int k = 0; k < PHX_PPT; ++k)
+      if (gi * PHX_CHUNK + threadIdx.x + k * PHX_BLOCK < e.n) {
+        if (k == 0) zblock_accumulate<0x05u>(v, p[k], zshift, minmax);
+        else zblock_accumulate<0u>(v, p[k], zshift, minmax);
+      }
+  }
+  double r[ZA_NV];
+#pragma unroll
+  for (int i = 0; i < ZA_NV; ++i) r[i] = v[za_slot(i)];
+  const double t = block_reduce_slots<ZA_NV, ZA_MINM, ZA_MAXM>(r, pass_lds);
+  if (threadIdx.x < ZA_NV) w.partials[(size_t)za_slot(threadIdx.x) * a.grid + bid] = t;
+}
+
+__device__ __forceinline__ void ahead_start_fold(const EngineArgs &a) {
+  const phx_engine &e = a.e;
+  __shared__ double res[ZB_NV];
+  EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
+  const int turn = *e.turn_counter;
+  const phx_turn_program &g = e.programs[e.turn_program[turn]];
+  AheadState &h = w.ahead[turn & 1];
+  if (threadIdx.x < 6) w.p0[threadIdx.x] = e.coords[threadIdx.x][0];
+  ahead_fold(w.partials, a.grid, res);
+  if (threadIdx.x == 0) {
+    const int cap = e.hist->capacity, nf = e.hist->n_filled;
+    ahead_set(h, g.slicer, e.n, res, (e.hist->head + 1) % cap, nf + 1 < cap ? nf + 1 : cap);
+  } else if (threadIdx.x == PHX_WAVE) {
+    h.zshift = ahead_shift(e.coords, g);
+  }
 }
 
 // The pass of space-charge stage `stage` > 0: the space-charge kick that
@@ -510,10 +788,9 @@ __device__ __forceinline__ void sc_pass_body(
   ScCtx scc;
   scc.sl = sw.slices;
   scc.wc = sw.wc;
-  scc.tail = sw.state->tail;
-  scc.width = sw.state->width;
-  scc.inv_width = 1.0 / scc.width;
-  scc.S = sw.state->n_slices;
+  scc.bins = SliceBins(sw.state->tail, sw.state->width, sw.state->n_slices);
+  // the cuts after this stage: its space-charge slicing's, or the wake's
+  const bool minmax = (g.has_sc ? g.sc_slicer : g.slicer).cuts_mode == PHX_CUTS_MINMAX;
   // particle 0's z after this stage's elements: the shift of the z sums
   double zshift;
   {
@@ -551,7 +828,7 @@ __device__ __forceinline__ void sc_pass_body(
           z[j] = p[0].z;
           st_mom(dp + j, p[0].dp);
         }
-        zblock_accumulate<0x05u>(v, p[0], zshift);
+        zblock_accumulate<0x05u>(v, p[0], zshift, minmax);
       }
     }
   }
@@ -662,9 +939,8 @@ __device__ __forceinline__ void hist_body(const EngineArgs &a, int bid, int nblk
   }
   AccLds A = acc_lds_layout(acc_lds, S, 2);
   acc_lds_zero(A, S, 2);  // ends with a barrier: the shared cuts are visible
-  const double tail = sh_st.tail, width = sh_st.width;
-  const double inv_width = 1.0 / width;
-  const int ex = fx_exponent(sh_st.absmax[0]), ey = fx_exponent(sh_st.absmax[2]);
+  const SliceBins bins(sh_st.tail, sh_st.width, S);
+  const FxScale fx = fx_scale(sh_st.absmax[0], n), fy = fx_scale(sh_st.absmax[2], n);
   load_chunk(bid, zz, xx, yy);
   for (int64_t c = bid; c < nc; c += nblk) {
     load_chunk(c + nblk, zn, xn, yn);
@@ -673,12 +949,11 @@ __device__ __forceinline__ void hist_body(const EngineArgs &a, int bid, int nblk
     for (int k = 0; k < EN_HIST_PPT; ++k) {
       const int64_t j = base + (int64_t)k * EN_HIST_THREADS;
       if (j < n) {
-        const double f = slice_floor_r(zz[k], tail, width, inv_width);
-        if (f >= 0.0 && f < (double)S) {
-          const int s = (int)f;
+        const int s = bins.index(zz[k]);
+        if (s >= 0) {
           atomicAdd(&A.counts[s], 1u);
-          acc_add_value(A, S, 0, s, xx[k], ex, w.acc.fallback);
-          acc_add_value(A, S, 1, s, yy[k], ey, w.acc.fallback);
+          acc_add_value(A, S, 0, s, xx[k], fx, w.acc.fallback);
+          acc_add_value(A, S, 1, s, yy[k], fy, w.acc.fallback);
         }
       }
     }
@@ -698,6 +973,46 @@ __device__ __forceinline__ void hist_body(const EngineArgs &a, int bid, int nblk
 // Block (S + SL - 1) / SL, launched when the engine has resistive-wall kicks
 // in the dot-product form, describes the turn's kicks for the convolution
 // (rw_desc_build) while the others merge.
+// Three-launch turns (ahead): the blocks after those fold the pass's z sums
+// into the next turn's cuts and do the bookkeeping that the histogram's block
+// 0 does in the four-launch turn (the merge blocks read the ring's new slot
+// from the turn's AheadState, so that nothing they read is written here).
+enum { MA_CUTS = 0, MA_SHIFT, MA_RING, MA_STATS, MA_STATS_BLOCKS = 4 };
+#define MA_THREADS 512
+__host__ __device__ inline int merge_blocks(int S, int SL, bool desc, bool ahead, bool rec) {
+  return (S + SL - 1) / SL + (desc ? 1 : 0) +
+         (ahead ? MA_STATS + (rec ? MA_STATS_BLOCKS : 0) : 0);
+}
+
+__device__ __forceinline__ void merge_slice(const phx_engine &e, const EngineWs &w, int s,
+                                            const SliceTotals &tot, int turn, double tail,
+                                            double width, double absx, double absy, int nh) {
+  const int S = e.n_slices;
+  // bin edges as np.arange(tail, head + 1e-7*width, width)
+  e.z_bins[s] = arange_value(tail, width, s);
+  if (s == S - 1) e.z_bins[S] = arange_value(tail, width, S);
+  const phx_turn_program &g = e.programs[e.turn_program[turn]];
+  const FxScale fx = fx_scale(absx, e.n), fy = fx_scale(absy, e.n);
+  const double cnt = (double)tot.count;
+  const double sx = fx_value(tot.hi[0], tot.lo[0], w.acc.fallback[s], fx);
+  const double sy = fx_value(tot.hi[1], tot.lo[1], w.acc.fallback[S + s], fy);
+  w.acc.fallback[s] = 0.0;
+  w.acc.fallback[S + s] = 0.0;
+  const double mx = tot.count ? sx / cnt : 0.0;
+  const double my = tot.count ? sy / cnt : 0.0;
+  e.counts[s] = (int32_t)tot.count;
+  e.slice_means[s] = mx;
+  e.slice_means[S + s] = my;
+  phx_wake_hist *h = e.hist;
+  const double zl = arange_value(tail, width, s), zr = arange_value(tail, width, s + 1);
+  const double zc = zl + 0.5 * (zr - zl);
+  h->times[(size_t)nh * S + s] = zc / g.beta_c;
+  double *mm = h->mom + (size_t)nh * 3 * S;
+  mm[s] = cnt;
+  mm[S + s] = cnt * mx;
+  mm[2 * S + s] = cnt * my;
+}
+
 template <int SL>
 __device__ __forceinline__ void merge_body(const EngineArgs &a, int bid) {
   const phx_engine &e = a.e;
@@ -708,39 +1023,94 @@ __device__ __forceinline__ void merge_body(const EngineArgs &a, int bid) {
   if (bid == (S + SL - 1) / SL) {
     if (a.n_kicks < 1 || !e.hist) return;
     const phx_turn_program &g = e.programs[e.turn_program[turn]];
-    rw_desc_build(e.hist, *reinterpret_cast<const WakeKicks *>(g.kick), a.n_kicks, a.T,
-                  engine_rw_desc(w, a.n_kicks, S, a.T));
+    const phx_wake_hist *h = e.hist;
+    rw_desc_build(h, *reinterpret_cast<const WakeKicks *>(g.kick), a.n_kicks, a.T,
+                  engine_rw_desc(w, a.n_kicks, S, a.T), h->n_filled, h->head, h->beta[h->head]);
     return;
   }
   if (bid == 0 && threadIdx.x == 0) *e.turn_counter = turn + 1;
   if (!acc_merge<2, SL>(w.acc, S, tot, bid)) return;
-  const int s = bid * SL + threadIdx.x % SL;
-  // bin edges as np.arange(tail, head + 1e-7*width, width)
-  const double tail = e.state->tail, width = e.state->width;
-  e.z_bins[s] = arange_value(tail, width, s);
-  if (s == S - 1) e.z_bins[S] = arange_value(tail, width, S);
+  merge_slice(e, w, bid * SL + threadIdx.x % SL, tot, turn, e.state->tail, e.state->width,
+              e.state->absmax[0], e.state->absmax[2], e.hist->head);
+}
+
+// The cuts of the next turn and this turn's published state.
+__device__ __forceinline__ void ahead_cuts_block(const EngineArgs &a, const EngineWs &w,
+                                                 int turn) {
+  const phx_engine &e = a.e;
+  __shared__ double res[ZB_NV];
   const phx_turn_program &g = e.programs[e.turn_program[turn]];
-  const int ex = fx_exponent(e.state->absmax[0]);
-  const int ey = fx_exponent(e.state->absmax[2]);
-  const double cnt = (double)tot.count;
-  const double sx = fx_value(tot.hi[0], tot.lo[0], ex) + w.acc.fallback[s];
-  const double sy = fx_value(tot.hi[1], tot.lo[1], ey) + w.acc.fallback[S + s];
-  w.acc.fallback[s] = 0.0;
-  w.acc.fallback[S + s] = 0.0;
-  const double mx = tot.count ? sx / cnt : 0.0;
-  const double my = tot.count ? sy / cnt : 0.0;
-  e.counts[s] = (int32_t)tot.count;
-  e.slice_means[s] = mx;
-  e.slice_means[S + s] = my;
-  phx_wake_hist *h = e.hist;
-  const int nh = h->head;
-  const double zl = arange_value(tail, width, s), zr = arange_value(tail, width, s + 1);
-  const double zc = zl + 0.5 * (zr - zl);
-  h->times[(size_t)nh * S + s] = zc / g.beta_c;
-  double *mm = h->mom + (size_t)nh * 3 * S;
-  mm[s] = cnt;
-  mm[S + s] = cnt * mx;
-  mm[2 * S + s] = cnt * my;
+  const AheadState &h = w.ahead[turn & 1];
+  const int cap = e.hist->capacity;
+  ahead_fold(w.partials, a.grid, res);
+  if (threadIdx.x == 0) {
+    phx_slice_state st;
+    st.tail = h.tail;
+    st.head = h.head;
+    st.width = h.width;
+    st.mean_z = h.mean_z;
+    st.sigma_z = h.sigma_z;
+    for (int i = 0; i < 6; ++i) st.absmax[i] = -INFINITY;
+    st.absmax[0] = res[5];
+    st.absmax[2] = res[7];
+    st.n = e.n;
+    st.n_slices = g.slicer.n_slices;
+    st.turn = turn;
+    st.valid = 1;
+    st.pad = 0;
+    *e.state = st;
+    ahead_set(w.ahead[(turn & 1) ^ 1], g.slicer, e.n, res, (h.nh + 1) % cap,
+              h.nf + 1 < cap ? h.nf + 1 : cap);
+    *e.turn_counter = turn + 1;
+  }
+}
+
+template <int SL>
+__device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
+  const phx_engine &e = a.e;
+  EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
+  const int S = e.n_slices;
+  const int turn = *w.cur_turn;
+  const AheadState &h = w.ahead[turn & 1];
+  const int nm = (S + SL - 1) / SL;
+  if (bid >= nm) {
+    const phx_turn_program &g = e.programs[e.turn_program[turn]];
+    const int k = bid - nm;
+    if (k == MA_CUTS) {
+      ahead_cuts_block(a, w, turn);
+    } else if (k == MA_SHIFT) {
+      if (threadIdx.x < 6) w.p0[threadIdx.x] = e.coords[threadIdx.x][0];
+      if (threadIdx.x == PHX_WAVE) w.ahead[(turn & 1) ^ 1].zshift = ahead_shift(e.coords, g);
+    } else if (k == MA_RING) {
+      // the stored entries age by the turn's increment; the new one (slot
+      // h.nh) has age 0 (WakeField.track, impedances/wakes.py:134-142)
+      phx_wake_hist *r = e.hist;
+      for (int i = threadIdx.x; i < h.nf; i += blockDim.x) {
+        const int sl = ring_slot(h.nh, i, r->capacity);
+        r->age[sl] = i == 0 ? 0.0 : r->age[sl] + g.age_increment;
+      }
+      if (threadIdx.x == 0) {
+        r->head = h.nh;
+        r->n_filled = h.nf;
+        r->beta[h.nh] = g.beta;
+      }
+    } else if (e.record_stats && k < MA_STATS + MA_STATS_BLOCKS) {
+      __shared__ double st[EN_NV];
+      constexpr int per = (EN_STAT_NV + MA_STATS_BLOCKS - 1) / MA_STATS_BLOCKS;
+      const int i0 = ZB_NV + (k - MA_STATS) * per;
+      const int i1 = i0 + per < EN_NV ? i0 + per : EN_NV;
+      fold_partials<0ULL, 0ULL>(w.partials, a.grid, i0, i1, st);
+      if (threadIdx.x < i1 - i0)
+        e.stats[(size_t)turn * EN_STAT_NV + (i0 - ZB_NV) + threadIdx.x] = st[i0 + threadIdx.x];
+    } else {
+      rw_desc_build(e.hist, *reinterpret_cast<const WakeKicks *>(g.kick), a.n_kicks, a.T,
+                    engine_rw_desc(w, a.n_kicks, S, a.T), h.nf, h.nh, g.beta);
+    }
+    return;
+  }
+  SliceTotals tot;
+  if (!acc_merge<2, SL, MA_THREADS>(ahead_parts(w, S, a.hblk), S, tot, bid)) return;
+  merge_slice(e, w, bid * SL + threadIdx.x % SL, tot, turn, h.tail, h.width, h.absx, h.absy, h.nh);
 }
 
 // Space-charge slicing of the state after stage `stage` (the slicing that
@@ -776,11 +1146,10 @@ __device__ __forceinline__ void sc_hist_body(const EngineArgs &a, int stage, int
   if (bid == 0 && threadIdx.x < 6) w.p0[threadIdx.x] = e.coords[threadIdx.x][0];
   AccLds A = acc_lds_layout(acc_lds, S, SC_TERMS);
   acc_lds_zero(A, S, SC_TERMS);  // ends with a barrier: the shared cuts are visible
-  const double tail = sh_st.tail, width = sh_st.width;
-  const double inv_width = 1.0 / width;
+  const SliceBins bins(sh_st.tail, sh_st.width, S);
   const double bx = sh_st.absmax[0], by = sh_st.absmax[2];
-  const int ex = fx_exponent(bx), ey = fx_exponent(by);
-  const int exx = fx_exponent(bx * bx), eyy = fx_exponent(by * by);
+  const FxScale fx = fx_scale(bx, n), fy = fx_scale(by, n);
+  const FxScale fxx = fx_scale(bx * bx, n), fyy = fx_scale(by * by, n);
   constexpr int CH = EN_HIST_THREADS * EN_HIST_PPT;
   const int64_t nc = (n + CH - 1) / CH;
   double zz[EN_HIST_PPT], xx[EN_HIST_PPT], yy[EN_HIST_PPT];
@@ -809,14 +1178,13 @@ __device__ __forceinline__ void sc_hist_body(const EngineArgs &a, int stage, int
     for (int k = 0; k < EN_HIST_PPT; ++k) {
       const int64_t j = base + (int64_t)k * EN_HIST_THREADS;
       if (j < n) {
-        const double f = slice_floor_r(zz[k], tail, width, inv_width);
-        if (f >= 0.0 && f < (double)S) {
-          const int s = (int)f;
+        const int s = bins.index(zz[k]);
+        if (s >= 0) {
           atomicAdd(&A.counts[s], 1u);
-          acc_add_value(A, S, 0, s, xx[k], ex, P.fallback);
-          acc_add_value(A, S, 1, s, yy[k], ey, P.fallback);
-          acc_add_value(A, S, 2, s, xx[k] * xx[k], exx, P.fallback);
-          acc_add_value(A, S, 3, s, yy[k] * yy[k], eyy, P.fallback);
+          acc_add_value(A, S, 0, s, xx[k], fx, P.fallback);
+          acc_add_value(A, S, 1, s, yy[k], fy, P.fallback);
+          acc_add_value(A, S, 2, s, xx[k] * xx[k], fxx, P.fallback);
+          acc_add_value(A, S, 3, s, yy[k] * yy[k], fyy, P.fallback);
         }
       }
     }
@@ -830,21 +1198,21 @@ __device__ __forceinline__ void sc_hist_body(const EngineArgs &a, int stage, int
   acc_lds_store(A, S, SC_TERMS, P, bid);
 }
 
-// A fixed-point total as an unevaluated double-double hi + lo (exact):
-// the integer h*2^32 + l, h = hi_sum + (lo_sum >> 32), l = lo_sum mod 2^32,
-// times 2^-e.
+// A fixed-point total as an unevaluated double-double hi + lo: fx_value
+// before its last rounding, the out-of-range parts (if any) in lo.
 __device__ __forceinline__ void fx_value_dd(unsigned long long hi_sum, unsigned long long lo_sum,
-                                            int e, double &hi, double &lo) {
-  const long long h = (long long)hi_sum + (long long)(lo_sum >> 32);
+                                            double over, const FxScale &f, double &hi,
+                                            double &lo) {
+  const long long h = (long long)hi_sum + ((long long)lo_sum >> FX_LB);
   const double a = (double)h;
-  const long long r = h - (long long)a;  // |r| <= 2^10
-  const double A = ldexp(a, 32);
-  const double B = (double)(r * 4294967296LL + (long long)(lo_sum & 0xffffffffULL));
-  const double s = A + B;
-  const double bb = s - A;
-  const double t = (A - (s - bb)) + (B - bb);
-  hi = ldexp(s, -e);
-  lo = ldexp(t, -e);
+  const long long r = h - (long long)a;
+  const double b = (double)(r * (1LL << FX_LB) + (long long)(lo_sum & ((1ULL << FX_LB) - 1ULL))) *
+                   (1.0 / (double)(1LL << FX_LB));
+  const double s = a + b;
+  const double bb = s - a;
+  const double t = (a - (s - bb)) + (b - bb);
+  hi = s * f.unit;
+  lo = t * f.unit + over;
 }
 
 // (q - x^2/n) / (n - 1) from double-double totals x = sum u, q = sum u^2:
@@ -885,8 +1253,8 @@ __device__ __forceinline__ void sc_merge_body(const EngineArgs &a, int stage, in
   const phx_slice_state &st = *sw.state;
   const double tail = st.tail, width = st.width;
   const double bx = st.absmax[0], by = st.absmax[2];
-  const int ex = fx_exponent(bx), ey = fx_exponent(by);
-  const int exx = fx_exponent(bx * bx), eyy = fx_exponent(by * by);
+  const FxScale sfx = fx_scale(bx, e.n), sfy = fx_scale(by, e.n);
+  const FxScale sfxx = fx_scale(bx * bx, e.n), sfyy = fx_scale(by * by, e.n);
   const double cnt = (double)tot.count;
   const double fx = P.fallback[s], fy = P.fallback[S + s];
   const double fxx = P.fallback[2 * S + s], fyy = P.fallback[3 * S + s];
@@ -894,20 +1262,20 @@ __device__ __forceinline__ void sc_merge_body(const EngineArgs &a, int stage, in
   P.fallback[S + s] = 0.0;
   P.fallback[2 * S + s] = 0.0;
   P.fallback[3 * S + s] = 0.0;
-  const double sx = fx_value(tot.hi[0], tot.lo[0], ex) + fx;
-  const double sy = fx_value(tot.hi[1], tot.lo[1], ey) + fy;
+  const double sx = fx_value(tot.hi[0], tot.lo[0], fx, sfx);
+  const double sy = fx_value(tot.hi[1], tot.lo[1], fy, sfy);
   ScSlice row;
   row.mx = tot.count ? sx / cnt : 0.0;
   row.my = tot.count ? sy / cnt : 0.0;
   double sgx = 0.0, sgy = 0.0;
   if (tot.count > 1) {
     double xh, xl, yh, yl, qxh, qxl, qyh, qyl;
-    fx_value_dd(tot.hi[0], tot.lo[0], ex, xh, xl);
-    fx_value_dd(tot.hi[1], tot.lo[1], ey, yh, yl);
-    fx_value_dd(tot.hi[2], tot.lo[2], exx, qxh, qxl);
-    fx_value_dd(tot.hi[3], tot.lo[3], eyy, qyh, qyl);
-    sgx = sqrt(var_from_sums(xh, xl + fx, qxh, qxl + fxx, cnt));
-    sgy = sqrt(var_from_sums(yh, yl + fy, qyh, qyl + fyy, cnt));
+    fx_value_dd(tot.hi[0], tot.lo[0], fx, sfx, xh, xl);
+    fx_value_dd(tot.hi[1], tot.lo[1], fy, sfy, yh, yl);
+    fx_value_dd(tot.hi[2], tot.lo[2], fxx, sfxx, qxh, qxl);
+    fx_value_dd(tot.hi[3], tot.lo[3], fyy, sfyy, qyh, qyl);
+    sgx = sqrt(var_from_sums(xh, xl, qxh, qxl, cnt));
+    sgy = sqrt(var_from_sums(yh, yl, qyh, qyl, cnt));
   }
   row.nl = sc_line_density((int32_t)tot.count, g.sc.charge_per_mp, arange_value(tail, width, s),
                            arange_value(tail, width, s + 1));

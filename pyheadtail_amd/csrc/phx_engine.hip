@@ -17,11 +17,15 @@
 //   4. wake convolution over the history (and, with several turns of memory,
 //      the in-order sum over turns).
 // Without a wake field a turn is the pass and a one-block finalize.
+// Sequences of turns of the same program are three launches per turn where
+// that applies (ahead_body in phx_engine.h): the pass slices the particles
+// itself and the merge folds the cuts.
 // No stage uses cross-block atomics or fences: kernel boundaries order the
 // stages, which keeps every reduction deterministic and avoids the
 // serialisation of device-scope atomics.  The kick of turn t is applied in
 // pass 1 of turn t+1, which gives the arithmetic of WakeField.track at the
 // end of turn t (impedances/wakes.py:121-145).
+#include "phx_ahead.h"
 #include "phx_engine.h"
 #include "phx_host.h"
 
@@ -96,9 +100,8 @@ __global__ void __launch_bounds__(PHX_BLOCK) k_engine_kick(EngineArgs a) {
   const int turn = *e.turn_counter;
   const phx_turn_program &g = e.programs[e.turn_program[turn > 0 ? turn - 1 : 0]];
   const int nk = g.n_kicks < a.n_kicks ? g.n_kicks : a.n_kicks;
-  const double tail = e.state->tail, width = e.state->width;
-  const double inv_width = 1.0 / width;
   const int S = e.n_slices;
+  const SliceBins bins(e.state->tail, e.state->width, S);
   double *const *c = e.coords;
   for (int64_t j = blockIdx.x * (int64_t)PHX_BLOCK + threadIdx.x; j < e.n;
        j += (int64_t)gridDim.x * PHX_BLOCK) {
@@ -109,9 +112,9 @@ __global__ void __launch_bounds__(PHX_BLOCK) k_engine_kick(EngineArgs a) {
     p.x = KS == PHX_KICKS_DXDY ? 0.0 : c[0][j];
     p.y = KS == PHX_KICKS_DXDY ? 0.0 : c[2][j];
     p.dp = KS == PHX_KICKS_GENERIC ? c[5][j] : 0.0;
-    const double f = slice_floor_r(p.z, tail, width, inv_width);
-    if (f >= 0.0 && f < (double)S) {
-      apply_kick_set<KS>(p, (int32_t)f, S, g.kick, nk, e.kicks);
+    const int s = bins.index(p.z);
+    if (s >= 0) {
+      apply_kick_set<KS>(p, s, S, g.kick, nk, e.kicks);
       c[1][j] = p.xp;
       c[3][j] = p.yp;
       if (KS == PHX_KICKS_GENERIC) c[5][j] = p.dp;
@@ -423,8 +426,13 @@ int scpass_blocks_per_cu(const phx_engine &e) {
 
 EngineArgs make_args(const phx_engine *e, int nk, int T) {
   const bool has_wake = e->n_slices > 0 && nk > 0;
-  EngineArgs a{*e, nk, T, 1, 1};
-  if (e->sc_stages > 0 && e->pass_grid == 0) {
+  EngineArgs a{*e, nk, T, 1, 1, 0, 0};
+  const bool fits = ahead_fits(*e);
+  if (fits && e->pass_grid == 0) {
+    // the four-launch turns of such an engine (short sequences, changing
+    // programs) share the grid, so that the cuts do not depend on which run
+    a.grid = phx_grid_for(e->n, (int64_t)ahead_max_nsub(*e) * phx_num_cus());
+  } else if (e->sc_stages > 0 && e->pass_grid == 0) {
     // every pass of a turn shares the grid (the partials' layout); space-
     // charge engines take the one that fills the device with their stage
     // passes, which carry most of the work
@@ -435,6 +443,16 @@ EngineArgs make_args(const phx_engine *e, int nk, int T) {
     a.grid = pass_grid(*e, pick_pass<0>(*e, has_wake || e->sc_stages > 0));
   }
   if (e->n_slices > 0) a.gmax = wake_conv_gmax(e->n_slices, phx_max_lds_bytes());
+  if (fits && e->ahead) {
+    // as many groups per block as leave at most one block per CU: bunches of
+    // up to a CU's worth of groups each spread over the CUs, one group each
+    const int cus = phx_num_cus(), most = ahead_max_nsub(*e);
+    a.nsub = (a.grid + cus - 1) / cus;
+    a.nsub = a.nsub < most ? a.nsub : most;
+    a.hblk = (a.grid + a.nsub - 1) / a.nsub;
+    const int hb = hist_blocks(e->n);
+    a.hblk = a.hblk < hb ? a.hblk : hb;
+  }
   return a;
 }
 
@@ -503,11 +521,10 @@ int enqueue_stage(const EngineArgs &a, int stage, bool has_wake, hipStream_t s) 
       k_engine_hist<false><<<dim3(hist_blocks(e.n)), EN_HIST_THREADS, acc_lds_bytes(e.n_slices, 2), s>>>(a);
     PHX_CHECK_LAUNCH("phx_engine: hist");
     // one more block describes the resistive-wall kicks for the convolution
-    const int desc = has_wake && engine_has_rw(e) ? 1 : 0;
-    if (merge_sl(e.n_slices) == 4)
-      k_engine_merge<4><<<dim3((e.n_slices + 3) / 4 + desc), PHX_BLOCK, 0, s>>>(a);
-    else
-      k_engine_merge<8><<<dim3((e.n_slices + 7) / 8 + desc), PHX_BLOCK, 0, s>>>(a);
+    const int sl = merge_sl(e.n_slices);
+    const dim3 grid((unsigned)merge_blocks(e.n_slices, sl, has_wake && engine_has_rw(e), false, false));
+    if (sl == 4) k_engine_merge<4><<<grid, PHX_BLOCK, 0, s>>>(a);
+    else k_engine_merge<8><<<grid, PHX_BLOCK, 0, s>>>(a);
     PHX_CHECK_LAUNCH("phx_engine: merge");
     return PHX_OK;
   }
@@ -563,6 +580,15 @@ int enqueue_flush(const EngineArgs &a, hipStream_t s) {
   k_engine_fin<1, false><<<1, PHX_BLOCK, 0, s>>>(a);
   PHX_CHECK_LAUNCH("phx_engine: flush finalize");
   return PHX_OK;
+}
+
+// A turn of a sequence that ahead_enqueue_start began.
+int enqueue_ahead_turn(const EngineArgs &a, hipStream_t s) {
+  int rc = ahead_enqueue_pass(a, s);
+  if (rc) return rc;
+  rc = ahead_enqueue_merge(a, s);
+  if (rc) return rc;
+  return enqueue_stage(a, 2, true, s);
 }
 
 int enqueue_turn(const EngineArgs &a, bool has_wake, hipStream_t s) {
@@ -627,7 +653,10 @@ extern "C" int phx_engine_reset(const phx_engine *e, phx_stream_t stream) {
   return PHX_OK;
 }
 
-// n_turns turns, after a snapshot of particle 0 if snapshot is set.
+// n_turns turns, after a snapshot of particle 0 (and, for three-launch turns,
+// their start) if snapshot is set.  A sequence without one continues another
+// that had it.  The start costs two launches and a read of x, y, z and dp
+// (13 us at 1e6 macroparticles), less than PHX_AHEAD_MIN_TURNS turns gain.
 static int engine_turns(const phx_engine *e, int32_t n_turns, hipStream_t s, bool snapshot) {
   int nk, T;
   int rc = check_engine(e, &nk, &T);
@@ -637,12 +666,13 @@ static int engine_turns(const phx_engine *e, int32_t n_turns, hipStream_t s, boo
   if (rc) return rc;
   const bool has_wake = e->n_slices > 0 && nk > 0;
   EngineArgs a = make_args(e, nk, T);
+  const bool ahead = a.nsub > 0 && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
   if (snapshot && n_turns > 0) {
-    rc = enqueue_snapshot(a, s);
+    rc = ahead ? ahead_enqueue_start(a, s) : enqueue_snapshot(a, s);
     if (rc) return rc;
   }
   for (int t = 0; t < n_turns; ++t) {
-    rc = enqueue_turn(a, has_wake, s);
+    rc = ahead ? enqueue_ahead_turn(a, s) : enqueue_turn(a, has_wake, s);
     if (rc) return rc;
   }
   return PHX_OK;
@@ -659,9 +689,12 @@ extern "C" int phx_engine_stage(const phx_engine *e, int32_t stage, phx_stream_t
   rc = check_lds(e);
   if (rc) return rc;
   const bool has_wake = e->n_slices > 0 && nk > 0;
-  if (stage < 0 || stage > 2 || (stage > 0 && !has_wake))
-    return phx::fail(PHX_E_INVALID, "phx_engine_stage: bad stage %d", stage);
   EngineArgs a = make_args(e, nk, T);
+  if (stage < 0 || stage > 5 || (stage > 0 && !has_wake))
+    return phx::fail(PHX_E_INVALID, "phx_engine_stage: bad stage %d", stage);
+  if (a.nsub > 0 && stage == 3) return ahead_enqueue_pass(a, phx::as_stream(stream));
+  if (a.nsub > 0 && stage == 4) return ahead_enqueue_merge(a, phx::as_stream(stream));
+  if (stage > 2) stage -= 3;
   return enqueue_stage(a, stage, has_wake, phx::as_stream(stream));
 }
 
@@ -676,7 +709,9 @@ extern "C" int phx_engine_snapshot(const phx_engine *e, phx_stream_t stream) {
   int nk, T;
   int rc = check_engine(e, &nk, &T);
   if (rc) return rc;
-  return enqueue_snapshot(make_args(e, nk, T), phx::as_stream(stream));
+  const EngineArgs a = make_args(e, nk, T);
+  return a.nsub > 0 ? ahead_enqueue_start(a, phx::as_stream(stream))
+                    : enqueue_snapshot(a, phx::as_stream(stream));
 }
 
 // ---------------------------------------------------------------------------

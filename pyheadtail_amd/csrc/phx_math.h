@@ -1,8 +1,7 @@
 // FP64 sine and cosine for the particle maps.
 //
-// The phases of the maps are moderate: the RF phase h*2*pi*z/C stays within
-// a few radians of the bucket, the betatron phase 2*pi*(Q + dQ) within a few
-// hundred radians.  For |x| < 2^20 the argument is reduced by Cody and
+// The maps count their phases in turns (phx_turns_n below).  Arguments in
+// radians (the wake functions; a few hundred at most):  For |x| < 2^20 the argument is reduced by Cody and
 // Waite's method with pi/2 split into P1 + P2 + P3: P1 and P2 carry 33
 // significant bits, so k*P1 and k*P2 are exact for |k| < 2^20 and x - k*P1
 // is exact (both are multiples of ulp(x) there); the remainder
@@ -94,39 +93,148 @@ __host__ __device__ __forceinline__ double reduce(double x, double &r_lo, int &q
   return r;
 }
 
+// sin(2 pi r) = r T(r^2) and cos(2 pi r) = 1 + r^2 U(r^2) for |r| <= 1/8:
+// the polynomials that interpolate sin(2 pi sqrt(z))/sqrt(z) and
+// (cos(2 pi sqrt(z)) - 1)/z at the Chebyshev nodes of [0, 1/64] (degree 6,
+// formed in 70-digit arithmetic and rounded to double; within 3.5e-18
+// relative and 1.3e-19 absolute of the functions).
+constexpr double T0 = 0x1.921fb54442d18p+2;
+constexpr double T1 = -0x1.4abbce625be41p+5;
+constexpr double T2 = 0x1.466bc677587f8p+6;
+constexpr double T3 = -0x1.32d2cce2e5b18p+6;
+constexpr double T4 = 0x1.50782fda12c1ep+5;
+constexpr double T5 = -0x1.e30071afacecep+3;
+constexpr double T6 = 0x1.e3f38390face5p+1;
+constexpr double U1 = -0x1.3bd3cc9be45dep+4;
+constexpr double U2 = 0x1.03c1f081b5ac0p+6;
+constexpr double U3 = -0x1.55d3c7e3cb241p+6;
+constexpr double U4 = 0x1.e1f5068688d5ap+5;
+constexpr double U5 = -0x1.a6d1eef479ab9p+4;
+constexpr double U6 = 0x1.f9ce245c9b912p+2;
+constexpr double U7 = -0x1.b2f3eafeb9c45p+0;
+constexpr double TURNS_MAX = 0x1p40;
+constexpr double TWO_PI = 0x1.921fb54442d18p+2;
+constexpr double INV_TWO_PI = 1.0 / TWO_PI;
+constexpr double TWO_PI_REL = -0x1.678afae35cdd1p-55;  // TWO_PI / (2 pi) - 1
+
 __device__ __noinline__ double cos_library(double x) { return ::cos(x); }
 
 __device__ __noinline__ double sin_library(double x) { return ::sin(x); }
 
 }  // namespace phx_math
 
-// sin(x) and cos(x); within ~1 ulp for |x| < 2^20, the device library's
-// values beyond (and for NaN / infinity).
-__device__ __forceinline__ void phx_sincos(double x, double *sp, double *cp) {
-  if (!(fabs(x) < phx_math::REDUCE_MAX)) {
-    *sp = phx_math::sin_library(x);
-    *cp = phx_math::cos_library(x);
-    return;
+// -v where bit 1 of quadrant is set.
+__device__ __forceinline__ double phx_flip(double v, int quadrant) {
+  return __longlong_as_double(__double_as_longlong(v) ^
+                              ((long long)((unsigned)(quadrant & 2) << 30) << 32));
+}
+
+// sin(x_k) and cos(x_k) of M arguments; within ~1 ulp for |x| < 2^20, the
+// device library's values beyond (and for NaN / infinity).  The M reductions
+// and polynomials run in lockstep (2 M independent chains of dependent FP64
+// operations, which the compiler interleaves), with one branch for arguments
+// out of range after all of them: a branch per argument keeps each chain in a
+// basic block of its own, and a wave then waits for one chain at a time.
+template <int M>
+__device__ __forceinline__ void phx_sincos_n(const double (&x)[M], double (&sp)[M],
+                                             double (&cp)[M]) {
+  bool far = false;
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    int q;
+    double r_lo, s, c;
+    const double r = phx_math::reduce(x[k], r_lo, q);
+    phx_math::kernel_sincos(r, r_lo, s, c);
+    // quadrant q: (sin, cos) = (s, c), (c, -s), (-s, -c), (-c, s)
+    sp[k] = phx_flip((q & 1) ? c : s, q);
+    cp[k] = phx_flip((q & 1) ? s : c, q + 1);
+    far |= !(fabs(x[k]) < phx_math::REDUCE_MAX);
   }
-  int q;
-  double r_lo;
-  const double r = phx_math::reduce(x, r_lo, q);
-  double s, c;
-  phx_math::kernel_sincos(r, r_lo, s, c);
-  // quadrant q: (sin, cos) = (s, c), (c, -s), (-s, -c), (-c, s)
-  const double sa = (q & 1) ? c : s;
-  const double ca = (q & 1) ? s : c;
-  *sp = (q & 2) ? -sa : sa;
-  *cp = ((q + 1) & 2) ? -ca : ca;
+  if (__builtin_expect(far, 0)) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      if (fabs(x[k]) < phx_math::REDUCE_MAX) continue;
+      sp[k] = phx_math::sin_library(x[k]);
+      cp[k] = phx_math::cos_library(x[k]);
+    }
+  }
+}
+
+// Sine and cosine of the maps' phases, counted in turns: u minus its nearest
+// quarter is exact, so no multiple of pi has to be subtracted in parts and the
+// reduced argument has no tail.  The quarter is rounded off by adding
+// 1.5 * 2^52, whose sum's low bits are the quadrant.  |u| >= 2^40 (and NaN,
+// infinity) go to the library.
+// COS (the betatron phases): sin(t) and cos(t) of t = u * (2.*np.pi) as the
+// reference rounds it; its distance from 2 pi u (up to 7e-15 rad by the
+// product's rounding and 5e-15 by the constant's at a tune of 20, ten times
+// what the rest of a segment map rounds) is put back after the reduction,
+// with three operations.  33 operations a pair against 45 with the reduction
+// in radians.  Otherwise (RF phases) sin(2 pi u) alone.
+template <int M, bool COS>
+__device__ __forceinline__ void phx_turns_n(const double (&u)[M], double (&sp)[M],
+                                            double (&cp)[M]) {
+  using namespace phx_math;
+  bool far = false;
+#pragma unroll
+  for (int k = 0; k < M; ++k) {
+    const double t = fma(u[k], 4.0, 0x1.8p52);
+    const int q = (int)__double_as_longlong(t);
+    double r = fma(t - 0x1.8p52, -0.25, u[k]);
+    if constexpr (COS) {
+      const double th = u[k] * TWO_PI;
+      r = fma(u[k], TWO_PI_REL, r);
+      r = fma(fma(u[k], TWO_PI, -th), -INV_TWO_PI, r);
+    }
+    const double z = r * r;
+    double ps = fma(T6, z, T5);
+    ps = fma(ps, z, T4);
+    ps = fma(ps, z, T3);
+    ps = fma(ps, z, T2);
+    ps = fma(ps, z, T1);
+    ps = fma(ps, z, T0);
+    double pc = fma(U7, z, U6);
+    pc = fma(pc, z, U5);
+    pc = fma(pc, z, U4);
+    pc = fma(pc, z, U3);
+    pc = fma(pc, z, U2);
+    pc = fma(pc, z, U1);
+    const double s = r * ps, c = fma(pc, z, 1.0);
+    sp[k] = phx_flip((q & 1) ? c : s, q);
+    if constexpr (COS) cp[k] = phx_flip((q & 1) ? s : c, q + 1);
+    far |= !(fabs(u[k]) < TURNS_MAX);
+  }
+  if (__builtin_expect(far, 0)) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      if (fabs(u[k]) < TURNS_MAX) continue;
+      sp[k] = sin_library(u[k] * TWO_PI);
+      if constexpr (COS) cp[k] = cos_library(u[k] * TWO_PI);
+    }
+  }
+}
+
+template <int M>
+__device__ __forceinline__ void phx_sincos_turns_n(const double (&u)[M], double (&sp)[M],
+                                                   double (&cp)[M]) {
+  phx_turns_n<M, true>(u, sp, cp);
+}
+
+template <int M>
+__device__ __forceinline__ void phx_sin_turns_n(const double (&u)[M], double (&sp)[M]) {
+  phx_turns_n<M, false>(u, sp, sp);
+}
+
+__device__ __forceinline__ void phx_sincos(double x, double *sp, double *cp) {
+  const double a[1] = {x};
+  double s[1], c[1];
+  phx_sincos_n<1>(a, s, c);
+  *sp = s[0];
+  *cp = c[0];
 }
 
 __device__ __forceinline__ double phx_sin(double x) {
-  if (!(fabs(x) < phx_math::REDUCE_MAX)) return phx_math::sin_library(x);
-  int q;
-  double r_lo;
-  const double r = phx_math::reduce(x, r_lo, q);
   double s, c;
-  phx_math::kernel_sincos(r, r_lo, s, c);
-  const double sa = (q & 1) ? c : s;
-  return (q & 2) ? -sa : sa;
+  phx_sincos(x, &s, &c);
+  return s;
 }

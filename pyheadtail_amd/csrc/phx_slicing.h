@@ -20,19 +20,29 @@ struct Coords6 {
 #define ZB_MINM (1ULL << 3)
 #define ZB_MAXM (0x7FULL << 4)
 
+// The slots that the fused engine's turns use (max |u| of x and y only), and
+// their place among those above.
+#define ZA_NV 7
+#define ZA_MINM (1ULL << 3)
+#define ZA_MAXM (0x7ULL << 4)
+__host__ __device__ constexpr int za_slot(int i) { return i < 6 ? i : 7; }
+
 // Bit i of AMASK: keep max |u_i| (the others stay -inf).  Comparisons
 // instead of fmin/fmax: the same results here (a NaN z or u never replaces
 // the running value, which is never NaN) without the NaN quieting of the
-// fmin/fmax instructions.
+// fmin/fmax instructions.  minmax (uniform): whether the cuts need min and
+// max z (PHX_CUTS_MINMAX).
 template <unsigned AMASK = 0x3Fu>
-__device__ __forceinline__ void zblock_accumulate(double (&v)[ZB_NV], const P6 &p,
-                                                  double shift) {
+__device__ __forceinline__ void zblock_accumulate(double (&v)[ZB_NV], const P6 &p, double shift,
+                                                  bool minmax) {
   const double dz = p.z - shift;
   v[0] = v[0] + p.z;
   v[1] = v[1] + dz;
-  v[2] = v[2] + dz * dz;
-  v[3] = p.z < v[3] ? p.z : v[3];
-  v[4] = p.z > v[4] ? p.z : v[4];
+  v[2] = fma(dz, dz, v[2]);
+  if (minmax) {
+    v[3] = p.z < v[3] ? p.z : v[3];
+    v[4] = p.z > v[4] ? p.z : v[4];
+  }
   const double a[6] = {fabs(p.x), fabs(p.xp), fabs(p.y), fabs(p.yp), fabs(p.z), fabs(p.dp)};
 #pragma unroll
   for (int i = 0; i < 6; ++i)
@@ -78,7 +88,7 @@ struct AccTerms {
 // merge block (one or two tiles) reads only whole cache lines of its own:
 //   cnt[tile][h][ACC_TW] (u32), hl[tile][h][t][ACC_TW] = {hi, lo} (u64
 //   pairs; one 128-byte line per tile and partial for t = 2),
-//   fallback[t][s] (f64, only for non-finite or out-of-scale values, merged
+//   fallback[t][s] (f64, only for non-finite or out-of-scale values, added
 //   with FP64 atomics).
 #define ACC_TW 4
 
@@ -128,7 +138,7 @@ __host__ __device__ inline AccParts acc_parts_layout(void *base, int H, int S, i
   return a;
 }
 
-inline size_t acc_lds_bytes(int S, int T) { return (size_t)T * S * 16 + (size_t)S * 4; }
+__host__ __device__ inline size_t acc_lds_bytes(int S, int T) { return (size_t)T * S * 16 + (size_t)S * 4; }
 
 __device__ __forceinline__ AccLds acc_lds_layout(unsigned long long *base, int S, int T) {
   AccLds L;
@@ -147,12 +157,14 @@ __device__ __forceinline__ void acc_lds_zero(const AccLds &L, int S, int T) {
   lds_sync();
 }
 
-// Bound of |term| from max|u| (centres are per-slice means, |c| <= max|u|).
-__device__ __forceinline__ int term_exponent(const AccTerms &t, int i, const double *absmax) {
+// The scale of a term's sums from max|u| (centres are per-slice means, |c| <=
+// max|u|).
+__device__ __forceinline__ FxScale term_scale(const AccTerms &t, int i, const double *absmax,
+                                              int64_t n) {
   double ba = absmax[t.a[i]] * (t.ca[i] ? 2.0 : 1.0);
   double bound = ba;
   if (t.b[i] >= 0) bound = ba * (absmax[t.b[i]] * (t.cb[i] ? 2.0 : 1.0));
-  return fx_exponent(bound);
+  return fx_scale(bound, n);
 }
 
 __device__ __forceinline__ double term_value(const AccTerms &t, int i, int s, const P6 &p) {
@@ -166,35 +178,37 @@ __device__ __forceinline__ double term_value(const AccTerms &t, int i, int s, co
   return u;
 }
 
-// True if u*2^e fits the fixed-point range; otherwise the value goes to the
-// FP64 fallback accumulator (non-finite values, or a bound that was violated).
-__device__ __forceinline__ bool fx_fits(double u, int e) {
-  const double q = ldexp(u, e);
-  return fabs(q) < 4611686018427387904.0;  // 2^62
-}
-
+// Adds u to sum i of slice s (every call adds one FX_MAGIC to both limbs).  A
+// value beyond the scale's range leaves its nearest multiple of lim in the
+// FP64 fallback (sums of such multiples are exact, so their order does not
+// matter either) and the rest in the limbs; a non-finite one goes to the
+// fallback as it is.
 __device__ __forceinline__ void acc_add_value(const AccLds &L, int S, int i, int s, double u,
-                                              int e, double *fallback) {
-  if (fx_fits(u, e)) {
-    unsigned long long hi, lo;
-    fx_split(u, e, hi, lo);
-    atomicAdd(&L.hi[(size_t)i * S + s], hi);
-    atomicAdd(&L.lo[(size_t)i * S + s], lo);
-  } else {
-    atomicAdd(&fallback[(size_t)i * S + s], u);
+                                              const FxScale &f, double *fallback) {
+  if (__builtin_expect(!(fabs(u) <= f.lim), 0)) {
+    double c = u;
+    if (fabs(u) < FX_HUGE) c = rint(u / f.lim) * f.lim;
+    atomicAdd(&fallback[(size_t)i * S + s], c);
+    u = fabs(u) < FX_HUGE ? u - c : 0.0;
   }
+  const double t = fma(u, f.s, FX_MAGIC);
+  const double r = fma(u, f.s, FX_MAGIC - t);  // u s - h, exact
+  const double l = fma(r, (double)(1LL << FX_LB), FX_MAGIC);
+  atomicAdd(&L.hi[(size_t)i * S + s], (unsigned long long)__double_as_longlong(t));
+  atomicAdd(&L.lo[(size_t)i * S + s], (unsigned long long)__double_as_longlong(l));
 }
 
 __device__ __forceinline__ void acc_add_lds(const AccLds &L, int S, const AccTerms &t,
-                                            const int *e, int s, const P6 &p,
+                                            const FxScale *f, int s, const P6 &p,
                                             double *fallback) {
   atomicAdd(&L.counts[s], 1u);
-  for (int i = 0; i < t.n; ++i) acc_add_value(L, S, i, s, term_value(t, i, s, p), e[i], fallback);
+  for (int i = 0; i < t.n; ++i) acc_add_value(L, S, i, s, term_value(t, i, s, p), f[i], fallback);
 }
 
 // Store this block's LDS histogram as partial number h (every entry, zeros
 // included, so the merge needs no prior clearing; the slots of a last,
-// partly used tile are never read).
+// partly used tile are never read): the limbs without their FX_MAGICs, the
+// low one reduced to FX_LB bits with its carry added to the high one.
 __device__ __forceinline__ void acc_lds_store(const AccLds &L, int S, int T, const AccParts &P,
                                               int h) {
   lds_sync();
@@ -206,9 +220,11 @@ __device__ __forceinline__ void acc_lds_store(const AccLds &L, int S, int T, con
     const int r = q % rec, i = r / ACC_TW;
     const int s = (q / rec) * ACC_TW + r % ACC_TW;
     if (s < S) {
+      const unsigned long long m = (unsigned long long)L.counts[s] * FX_MAGIC_BITS;
+      const long long lo = (long long)(L.lo[(size_t)i * S + s] - m);
       ulonglong2 v;
-      v.x = L.hi[(size_t)i * S + s];
-      v.y = L.lo[(size_t)i * S + s];
+      v.x = L.hi[(size_t)i * S + s] - m + (unsigned long long)(lo >> FX_LB);
+      v.y = (unsigned long long)lo & ((1ULL << FX_LB) - 1ULL);
       P.hl[acc_hl_index(P.H, T, h, i, s)] = v;
     }
   }
@@ -230,11 +246,12 @@ struct SliceTotals {
   unsigned long long hi[PHX_MAX_TERMS], lo[PHX_MAX_TERMS];
 };
 
-// bid: the tile of SL slices (blockIdx.x of the standalone launch)
-template <int T, int SL = RD_SL>
+// bid: the tile of SL slices (blockIdx.x of the standalone launch); NT: the
+// block's threads
+template <int T, int SL = RD_SL, int NT = PHX_BLOCK>
 __device__ __forceinline__ bool acc_merge(const AccParts &P, int S, SliceTotals &out, int bid) {
   constexpr int NVAL = 2 * T + 1;
-  constexpr int NW = PHX_BLOCK / PHX_WAVE;
+  constexpr int NW = NT / PHX_WAVE;
   __shared__ unsigned long long wsum[NW][NVAL][SL];
   const int sl = threadIdx.x % SL, g = threadIdx.x / SL;
   const int s = bid * SL + sl;
@@ -243,7 +260,7 @@ __device__ __forceinline__ bool acc_merge(const AccParts &P, int S, SliceTotals 
 #pragma unroll
   for (int i = 0; i < NVAL; ++i) v[i] = 0ULL;
   if (s < S) {
-    for (int h = g; h < P.H; h += (PHX_BLOCK / SL)) {
+    for (int h = g; h < P.H; h += (NT / SL)) {
       v[0] += P.cnt[acc_cnt_index(P.H, h, s)];
 #pragma unroll
       for (int i = 0; i < T; ++i) {

@@ -125,7 +125,7 @@ extern "C" int phx_bunch_sums(const double *const *arrays, int32_t k, int64_t n,
 // Slicing cuts: z sums of the current coordinates and max|u| of all six.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(PHX_BLOCK)
-    k_slice_cuts(Coords6 co, int64_t n, double *partials) {
+    k_slice_cuts(Coords6 co, int64_t n, double *partials, bool minmax) {
   __shared__ double lds[BR_LDS(ZB_NV)];
   const double shift = co.c[4][0];
   double v[ZB_NV];
@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(PHX_BLOCK)
       p.yp = co.c[3] ? co.c[3][j] : 0.0;
       p.z = co.c[4][j];
       p.dp = co.c[5] ? co.c[5][j] : 0.0;
-      zblock_accumulate(v, p, shift);
+      zblock_accumulate(v, p, shift, minmax);
     }
   }
   }
@@ -176,7 +176,8 @@ extern "C" int phx_slice_cuts(const double *const coords[6], int64_t n, const ph
   double *partials = reinterpret_cast<double *>(reinterpret_cast<char *>(ws) + phx::WsLayout::kTicketBytes);
   const int64_t nc = phx_pass_grid(n);
   hipStream_t s = phx::as_stream(stream);
-  k_slice_cuts<<<dim3((unsigned)nc), PHX_BLOCK, 0, s>>>(co, n, partials);
+  k_slice_cuts<<<dim3((unsigned)nc), PHX_BLOCK, 0, s>>>(co, n, partials,
+                                                         cfg->cuts_mode == PHX_CUTS_MINMAX);
   k_slice_cuts_fin<<<1, PHX_BLOCK, 0, s>>>(partials, nc, *cfg, n, state, z_bins);
   PHX_CHECK_LAUNCH("phx_slice_cuts");
   return PHX_OK;
@@ -198,8 +199,8 @@ __global__ void __launch_bounds__(PHX_BLOCK)
                        const int32_t *idx_in, int32_t *idx_out, AccParts P) {
   extern __shared__ unsigned long long acc_lds[];
   const double tail = state->tail, width = state->width;
-  int e[PHX_MAX_TERMS];
-  for (int t = 0; t < terms.n; ++t) e[t] = term_exponent(terms, t, state->absmax);
+  __shared__ FxScale f[PHX_MAX_TERMS];
+  if (threadIdx.x < terms.n) f[threadIdx.x] = term_scale(terms, threadIdx.x, state->absmax, n);
   AccLds L = acc_lds_layout(acc_lds, S, terms.n);
   acc_lds_zero(L, S, terms.n);
   const int64_t n_chunks = (n + PHX_CHUNK - 1) / PHX_CHUNK;
@@ -225,7 +226,7 @@ __global__ void __launch_bounds__(PHX_BLOCK)
           p.yp = co.c[3] ? co.c[3][j] : 0.0;
           p.z = z;
           p.dp = co.c[5] ? co.c[5][j] : 0.0;
-          acc_add_lds(L, S, terms, e, s, p, P.fallback);
+          acc_add_lds(L, S, terms, f, s, p, P.fallback);
         }
       }
     }
@@ -237,7 +238,7 @@ __global__ void __launch_bounds__(PHX_BLOCK)
 // re-zero the FP64 fallback entries.
 template <int T>
 __global__ void __launch_bounds__(RD_SL * RD_G)
-    k_slice_acc_merge(AccParts P, int S, AccTerms terms, const phx_slice_state *state,
+    k_slice_acc_merge(AccParts P, int S, AccTerms terms, const phx_slice_state *state, int64_t n,
                       int32_t *counts, double *sums, double *means) {
   SliceTotals tot;
   if (!acc_merge<T>(P, S, tot, blockIdx.x)) return;
@@ -245,9 +246,9 @@ __global__ void __launch_bounds__(RD_SL * RD_G)
   if (counts) counts[s] = (int32_t)tot.count;
 #pragma unroll
   for (int i = 0; i < T; ++i) {
-    const int e = term_exponent(terms, i, state->absmax);
     const size_t k = (size_t)i * S + s;
-    const double v = fx_value(tot.hi[i], tot.lo[i], e) + P.fallback[k];
+    const double v = fx_value(tot.hi[i], tot.lo[i], P.fallback[k],
+                              term_scale(terms, i, state->absmax, n));
     P.fallback[k] = 0.0;
     if (sums) sums[k] = v;
     if (means) means[k] = tot.count ? v / (double)tot.count : 0.0;
@@ -308,9 +309,9 @@ extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
   const dim3 mg((S + RD_SL - 1) / RD_SL);
   switch (n_terms) {
 #define PHX_MG(TT) \
-    case TT: k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, counts, sums, means); break;
+    case TT: k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means); break;
     PHX_MG(0) PHX_MG(1) PHX_MG(2) PHX_MG(3) PHX_MG(4) PHX_MG(5) PHX_MG(6) PHX_MG(7)
-    default: k_slice_acc_merge<8><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, counts, sums, means);
+    default: k_slice_acc_merge<8><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means);
 #undef PHX_MG
   }
   PHX_CHECK_LAUNCH("phx_slice_accumulate: merge");

@@ -711,10 +711,13 @@ __host__ __device__ inline const double *rw_desc_coef(const RwKick *d) {
   return reinterpret_cast<const double *>(d + PHX_MAX_KICKS);
 }
 
-// Builds the description of the nk kicks `table` over T turns of history h;
-// called by every thread of one block (any size).
+// Builds the description of the nk kicks `table` over T turns of history h
+// with nf entries, the newest in slot head with beta beta_head (the ring's own
+// may still be those of the turn before); called by every thread of one block
+// (any size).
 __device__ __forceinline__ void rw_desc_build(const phx_wake_hist *h, const WakeKicks &table,
-                                              int nk, int T, RwKick *d) {
+                                              int nk, int T, RwKick *d, int nf, int head,
+                                              double beta_head) {
   __shared__ WakeKicks kk;
   stage_kicks(table, nk, kk);
   if (threadIdx.x < nk) {
@@ -738,14 +741,14 @@ __device__ __forceinline__ void rw_desc_build(const phx_wake_hist *h, const Wake
     r.wake_factor = kw.wake_factor;
     d[k] = r;
   }
-  const int nf = h->n_filled, head = h->head, cap = h->capacity;
+  const int cap = h->capacity;
   double *coef = rw_desc_coef(d);
   for (int i = threadIdx.x; i < T * nk; i += blockDim.x) {
     const int t = i / nk, k = i % nk;
     const phx_wake_kick &kw = kk.k[k];
     double c = 0.0;
     if (t < nf && is_rw_dot(kw)) {
-      const double beta = h->beta[ring_slot(head, t, cap)];
+      const double beta = t == 0 ? beta_head : h->beta[ring_slot(head, t, cap)];
       c = (rw_prefix0(kw, beta) * sqrt(-kw.k_sigma)) * kw.sqrt_z0c;
     }
     coef[i] = c;

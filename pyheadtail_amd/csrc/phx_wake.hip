@@ -19,7 +19,7 @@ __global__ void __launch_bounds__(WK_THREADS)
 }
 
 __global__ void k_wake_rw_desc(const phx_wake_hist *h, WakeKicks kk, int nk, int T, RwKick *desc) {
-  rw_desc_build(h, kk, nk, T, desc);
+  rw_desc_build(h, kk, nk, T, desc, h->n_filled, h->head, h->beta[h->head]);
 }
 
 template <int KM>

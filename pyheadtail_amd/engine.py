@@ -1,5 +1,5 @@
-"""Fused one-turn map: many turns of [local elements..., WakeField] with four
-kernel launches per turn and no host synchronisation.
+"""Fused one-turn map: many turns of [local elements..., WakeField] with three
+or four kernel launches per turn and no host synchronisation.
 
 FusedOneTurnMap(one_turn_map) accepts the element list that a user would
 otherwise track one by one (as Synchrotron.one_turn_map,
@@ -394,8 +394,12 @@ class FusedOneTurnMap(Element):
                                      device=dev)
         return b
 
-    def _engine_record(self, beam, b, n_turns):
+    def _engine_record(self, beam, b, steady):
         eng = _phx.Engine()
+        # three-launch turns: one program for every turn from here on, and
+        # kicks (KICKS_DXDY, KICKS_PLATES) that leave z and dp alone
+        eng.ahead = 1 if (steady and not self.sc and self.wake is not None and
+                          self._shape[1] != _phx.KICKS_GENERIC) else 0
         for i, k in enumerate(COORDS):
             eng.coords[i] = beam._raw(k).data_ptr()
         eng.n = beam.macroparticlenumber
@@ -481,7 +485,11 @@ class FusedOneTurnMap(Element):
         if not np.array_equal(b['host_table'][:n_turns], table):
             b['table'][:n_turns].copy_(torch.from_numpy(table))
             b['host_table'][:n_turns] = table
-        eng = self._engine_record(beam, b, n_turns)
+        # the turns before the program settles (an RF kick re-derives p0 from
+        # gamma, which moves its last bit in the first turn) run one by one
+        moving = np.flatnonzero(np.diff(table))
+        self._unsteady = int(moving[-1]) + 1 if len(moving) else 0
+        eng = self._engine_record(beam, b, self._unsteady < n_turns)
         self._engine = eng
         if b.get('needs_reset'):
             _phx.call(L.phx_engine_reset, C.byref(eng), _phx.stream())
@@ -498,6 +506,16 @@ class FusedOneTurnMap(Element):
         elif self.record_stats:
             self._finish_stats(beam)
 
+    def _begin(self, eng, s, n_turns):
+        """Runs the first turns of a call where they need another launch
+        sequence than the rest; returns their number."""
+        k = self._unsteady if eng.ahead else 0
+        if k:
+            eng.ahead = 0
+            _phx.call(_phx.lib().phx_engine_turns, C.byref(eng), k, s)
+            eng.ahead = 1
+        return k
+
     def track_turns(self, beam, n_turns, use_graph=True):
         """Advance beam by n_turns turns."""
         if n_turns <= 0:
@@ -506,9 +524,9 @@ class FusedOneTurnMap(Element):
         eng = self._prepare(beam, n_turns)
         s = _phx.stream()
         G = self.graph_turns
-        done = 0
-        if use_graph and G > 0 and n_turns >= G:
-            key = (tuple(eng.coords), self.record_stats, G)
+        done = self._begin(eng, s, n_turns)
+        if use_graph and G > 0 and n_turns - done >= G:
+            key = (tuple(eng.coords), self.record_stats, G, self._shape, eng.ahead)
             h = self._graphs.get(key)
             if h is None:
                 h = C.c_void_p()
@@ -525,11 +543,14 @@ class FusedOneTurnMap(Element):
     def timed_turns(self, beam, n_turns):
         """Run n_turns with one launch per stage, bracketing every stage with
         HIP events on the launch stream; returns the mean duration of each
-        stage in ms (pass, histogram, convolution)."""
+        stage in ms: pass, histogram and merge, convolution; for three-launch
+        turns the pass with the slicing, the merge, the convolution."""
         L = _phx.lib()
         eng = self._prepare(beam, n_turns)
         s = _phx.stream()
         n_st = 3 if self.wake is not None else 1
+        first = 3 if eng.ahead else 0
+        n_turns -= self._begin(eng, s, n_turns)
         _phx.call(L.phx_engine_snapshot, C.byref(eng), s)
         ev = [[torch.cuda.Event(enable_timing=True) for _ in range(n_st + 1)]
               for _ in range(n_turns)]
@@ -540,7 +561,7 @@ class FusedOneTurnMap(Element):
         for t in range(n_turns):
             ev[t][0].record()
             for st in range(n_st):
-                _phx.call(L.phx_engine_stage, C.byref(eng), st, s)
+                _phx.call(L.phx_engine_stage, C.byref(eng), first + st, s)
                 ev[t][st + 1].record()
         torch.cuda.synchronize()
         self._finish(beam)
