@@ -121,7 +121,11 @@ class BatchedScan(object):
         recs = [eng._prepare(b, n_turns) for eng, b in zip(self.engines, self.bunches)]
         groups = {}
         for i, r in enumerate(recs):
-            groups.setdefault((r.record_stats, r.program_shape, r.det_shape), []).append(i)
+            # a batch's turns are three launches from the first turn or not
+            if self.engines[i]._unsteady:
+                r.ahead = 0
+            groups.setdefault((r.record_stats, r.program_shape, r.det_shape, r.ahead),
+                              []).append(i)
         if self._groups is None:
             self._groups = {}
         for key, idx in groups.items():

@@ -9,9 +9,12 @@
 // stage (the single-engine histogram folds them in every block).
 //   stages of a turn: pass | cuts | histogram | merge | convolution
 //   (general, resistive wall, resistive wall on the matrix cores) | sum over
-//   turns of memory; the empty ones are not launched.
+//   turns of memory; the empty ones are not launched.  Three-launch turns
+//   (every engine's ahead set and applicable): pass with slicing | merge |
+//   convolution...
 #include <vector>
 
+#include "phx_ahead.h"
 #include "phx_engine.h"
 #include "phx_host.h"
 
@@ -20,7 +23,14 @@ using namespace phx_en;
 namespace {
 
 enum { BS_PASS = 0, BS_CUTS, BS_HIST, BS_MERGE, BS_CONV, BS_RW, BS_RWMF, BS_RED, BS_SNAP,
-       BS_COUNT };
+       BS_APASS, BS_AMERGE, BS_COUNT };
+
+// Groups of threads per block of a batch's three-launch pass.  The single
+// engine's blocks fill a CU each, so that a CU stores one partial histogram;
+// a batch has many times the blocks that are resident, and blocks of one
+// group leave a CU several that start, compute and reduce at different times
+// (8 bunches of 1e6, 20 turns: 6046 us; two groups 6243, three 7576).
+#define PHX_BATCH_NSUB 1
 
 struct BatchArgs {
   const EngineArgs *args;  // [n] (device)
@@ -59,6 +69,44 @@ __global__ void __launch_bounds__(PHX_BLOCK) k_batch_pass(BatchArgs ba) {
   else
     pass_body<0, REC, true, SHAPE, PHX_KICKS_GENERIC, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5],
                                                           e.programs, e.kicks, loc, a.grid);
+}
+
+// The turn's map and the slicing of every engine.  Bound by its FP64
+// instructions (8 bunches of 1e6: 225 us, about 195 of them); the pass,
+// cuts and histogram launches that it replaces took 205 + 7 + 73 us.  The
+// compiler's own 180..300 registers (two blocks a CU) are the best choice:
+// forced to three blocks it spills (scan of 20 turns 9089 us against 6046).
+template <bool REC, int SHAPE, int DS>
+__global__ void __launch_bounds__(PHX_BLOCK) k_batch_ahead(BatchArgs ba) {
+  int loc;
+  const int b = batch_find(ba, BS_APASS, blockIdx.x, loc);
+  const EngineArgs &a = ba.args[b];
+  const phx_engine &e = a.e;
+  double *const *c = e.coords;
+  if (e.kick_shape == PHX_KICKS_DXDY)
+    ahead_body<REC, SHAPE, PHX_KICKS_DXDY, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5], e.programs,
+                                               e.kicks, loc, a.hblk, PHX_BATCH_NSUB);
+  else
+    ahead_body<REC, SHAPE, PHX_KICKS_PLATES, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5],
+                                                 e.programs, e.kicks, loc, a.hblk, PHX_BATCH_NSUB);
+}
+
+__global__ void __launch_bounds__(PHX_BLOCK) k_batch_ahead_start(BatchArgs ba) {
+  int loc;
+  const int b = batch_find(ba, BS_PASS, blockIdx.x, loc);
+  ahead_start_body(ba.args[b], loc);
+}
+
+__global__ void __launch_bounds__(PHX_BLOCK) k_batch_ahead_fold(BatchArgs ba) {
+  ahead_start_fold(ba.args[blockIdx.x]);
+}
+
+__global__ void __launch_bounds__(MA_THREADS) k_batch_ahead_merge(BatchArgs ba) {
+  int loc;
+  const int b = batch_find(ba, BS_AMERGE, blockIdx.x, loc);
+  const EngineArgs &a = ba.args[b];
+  if (merge_sl(a.e.n_slices) == 4) ahead_merge_body<4>(a, loc);
+  else ahead_merge_body<8>(a, loc);
 }
 
 template <bool REC>
@@ -117,7 +165,8 @@ struct Batch {
   int n;
   int rec, shape, dets;
   int total[BS_COUNT];
-  size_t lds_pass, lds_hist, lds_conv, lds_rw;
+  bool ahead;  // three-launch turns
+  size_t lds_pass, lds_hist, lds_conv, lds_rw, lds_ahead;
   void *desc;
   std::vector<char> host;  // the descriptor image, kept for the copy
   BatchArgs args() const {
@@ -149,6 +198,9 @@ void stage_blocks(const EngineArgs &a, int (&nb)[BS_COUNT]) {
   nb[BS_RWMF] = (ck == 0 || (ck & PHX_CONV_RW_MFMA)) ? rw_tiles * conv_rows(S, a.T) : 0;
   nb[BS_RED] = conv_reduces(S, a.T, engine_has_rw(e)) ? (a.n_kicks * S * RED_LANES + 255) / 256 : 0;
   nb[BS_SNAP] = 1;
+  nb[BS_APASS] = a.hblk;
+  nb[BS_AMERGE] = merge_blocks(S, merge_sl(S), has_wake && engine_has_rw(e), true,
+                               e.record_stats != 0);
 }
 
 // The compiled batch passes: first-order chromaticity (with or without
@@ -156,53 +208,63 @@ void stage_blocks(const EngineArgs &a, int (&nb)[BS_COUNT]) {
 // linear map, and the generic interpreter for every other map (and for
 // statistics records).
 template <bool REC, int SH, int DS>
-void launch_batch_pass(const Batch &B, hipStream_t s) {
+void launch_batch_pass(const Batch &B, bool ahead, hipStream_t s) {
+  if (ahead) {
+    k_batch_ahead<REC, SH, DS><<<dim3((unsigned)B.total[BS_APASS]), PHX_BATCH_NSUB * PHX_BLOCK,
+                                 B.lds_ahead, s>>>(B.args());
+    return;
+  }
   k_batch_pass<REC, SH, DS><<<dim3((unsigned)B.total[BS_PASS]), PHX_BLOCK, B.lds_pass, s>>>(
       B.args());
 }
 
 template <int SH>
-bool batch_pass_dets(const Batch &B, hipStream_t s) {
+bool batch_pass_dets(const Batch &B, bool ahead, hipStream_t s) {
   switch (B.dets) {
-    case PHX_DETS_C1: launch_batch_pass<false, SH, PHX_DETS_C1>(B, s); return true;
-    case PHX_DETS_C1_AMP: launch_batch_pass<false, SH, PHX_DETS_C1_AMP>(B, s); return true;
+    case PHX_DETS_C1: launch_batch_pass<false, SH, PHX_DETS_C1>(B, ahead, s); return true;
+    case PHX_DETS_C1_AMP: launch_batch_pass<false, SH, PHX_DETS_C1_AMP>(B, ahead, s); return true;
     case PHX_DETS_C1 | PHX_DETS_SMOOTH:
-      launch_batch_pass<false, SH, PHX_DETS_C1 | PHX_DETS_SMOOTH>(B, s);
+      launch_batch_pass<false, SH, PHX_DETS_C1 | PHX_DETS_SMOOTH>(B, ahead, s);
       return true;
     case PHX_DETS_C1_AMP | PHX_DETS_SMOOTH:
-      launch_batch_pass<false, SH, PHX_DETS_C1_AMP | PHX_DETS_SMOOTH>(B, s);
+      launch_batch_pass<false, SH, PHX_DETS_C1_AMP | PHX_DETS_SMOOTH>(B, ahead, s);
       return true;
     default: return false;
   }
 }
 
-int batch_pass(const Batch &B, hipStream_t s) {
+int batch_pass(const Batch &B, bool ahead, hipStream_t s) {
   bool done = false;
   if (B.rec) {
-    launch_batch_pass<true, PHX_SHAPE_GENERIC, PHX_DETS_GENERIC>(B, s);
+    launch_batch_pass<true, PHX_SHAPE_GENERIC, PHX_DETS_GENERIC>(B, ahead, s);
     done = true;
   } else if (B.shape == PHX_SHAPE_RF1_T) {
-    done = batch_pass_dets<PHX_SHAPE_RF1_T>(B, s);
+    done = batch_pass_dets<PHX_SHAPE_RF1_T>(B, ahead, s);
   } else if (B.shape == PHX_SHAPE_LIN_T) {
-    done = batch_pass_dets<PHX_SHAPE_LIN_T>(B, s);
+    done = batch_pass_dets<PHX_SHAPE_LIN_T>(B, ahead, s);
   }
-  if (!done) launch_batch_pass<false, PHX_SHAPE_GENERIC, PHX_DETS_GENERIC>(B, s);
+  if (!done) launch_batch_pass<false, PHX_SHAPE_GENERIC, PHX_DETS_GENERIC>(B, ahead, s);
   PHX_CHECK_LAUNCH("phx_batch: pass");
   return PHX_OK;
 }
 
-int batch_turn(const Batch &B, hipStream_t s) {
+int batch_turn(const Batch &B, bool ahead, hipStream_t s) {
   const BatchArgs ba = B.args();
-  int rc = batch_pass(B, s);
+  int rc = batch_pass(B, ahead, s);
   if (rc) return rc;
-  if (B.rec) k_batch_cuts<true><<<dim3(B.n), EN_HIST_THREADS, 0, s>>>(ba);
-  else k_batch_cuts<false><<<dim3(B.n), EN_HIST_THREADS, 0, s>>>(ba);
-  PHX_CHECK_LAUNCH("phx_batch: cuts");
-  if (B.rec) k_batch_hist<true><<<dim3(B.total[BS_HIST]), EN_HIST_THREADS, B.lds_hist, s>>>(ba);
-  else k_batch_hist<false><<<dim3(B.total[BS_HIST]), EN_HIST_THREADS, B.lds_hist, s>>>(ba);
-  PHX_CHECK_LAUNCH("phx_batch: histogram");
-  k_batch_merge<<<dim3(B.total[BS_MERGE]), PHX_BLOCK, 0, s>>>(ba);
-  PHX_CHECK_LAUNCH("phx_batch: merge");
+  if (ahead) {
+    k_batch_ahead_merge<<<dim3(B.total[BS_AMERGE]), MA_THREADS, 0, s>>>(ba);
+    PHX_CHECK_LAUNCH("phx_batch: merge");
+  } else {
+    if (B.rec) k_batch_cuts<true><<<dim3(B.n), EN_HIST_THREADS, 0, s>>>(ba);
+    else k_batch_cuts<false><<<dim3(B.n), EN_HIST_THREADS, 0, s>>>(ba);
+    PHX_CHECK_LAUNCH("phx_batch: cuts");
+    if (B.rec) k_batch_hist<true><<<dim3(B.total[BS_HIST]), EN_HIST_THREADS, B.lds_hist, s>>>(ba);
+    else k_batch_hist<false><<<dim3(B.total[BS_HIST]), EN_HIST_THREADS, B.lds_hist, s>>>(ba);
+    PHX_CHECK_LAUNCH("phx_batch: histogram");
+    k_batch_merge<<<dim3(B.total[BS_MERGE]), PHX_BLOCK, 0, s>>>(ba);
+    PHX_CHECK_LAUNCH("phx_batch: merge");
+  }
   if (B.total[BS_CONV]) {
     k_batch_conv<<<dim3(B.total[BS_CONV]), WK_THREADS, B.lds_conv, s>>>(ba);
     PHX_CHECK_LAUNCH("phx_batch: convolution");
@@ -222,13 +284,29 @@ int batch_turn(const Batch &B, hipStream_t s) {
   return PHX_OK;
 }
 
-int batch_turns(const Batch &B, int n_turns, hipStream_t s, bool snapshot) {
-  if (snapshot && n_turns > 0) {
+// Particle 0 of every engine or, for three-launch turns, their start.
+int batch_begin(const Batch &B, bool ahead, hipStream_t s) {
+  if (!ahead) {
     k_batch_snapshot<<<dim3(B.n), 64, 0, s>>>(B.args());
     PHX_CHECK_LAUNCH("phx_batch: snapshot");
+    return PHX_OK;
+  }
+  k_batch_ahead_start<<<dim3((unsigned)B.total[BS_PASS]), PHX_BLOCK, BR_LDS(ZA_NV) * sizeof(double),
+                        s>>>(B.args());
+  PHX_CHECK_LAUNCH("phx_batch: first turn's z sums");
+  k_batch_ahead_fold<<<dim3(B.n), PHX_BLOCK, 0, s>>>(B.args());
+  PHX_CHECK_LAUNCH("phx_batch: first turn's cuts");
+  return PHX_OK;
+}
+
+int batch_turns(const Batch &B, int n_turns, hipStream_t s, bool snapshot) {
+  const bool ahead = B.ahead && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
+  if (snapshot && n_turns > 0) {
+    const int rc = batch_begin(B, ahead, s);
+    if (rc) return rc;
   }
   for (int t = 0; t < n_turns; ++t) {
-    const int rc = batch_turn(B, s);
+    const int rc = batch_turn(B, ahead, s);
     if (rc) return rc;
   }
   return PHX_OK;
@@ -256,7 +334,8 @@ extern "C" int phx_batch_create(const phx_engine *engines, int32_t n, void *desc
   EngineArgs *args = reinterpret_cast<EngineArgs *>(B->host.data());
   int *off = reinterpret_cast<int *>(B->host.data() + round256((size_t)n * sizeof(EngineArgs)));
   for (int k = 0; k < BS_COUNT; ++k) B->total[k] = 0;
-  B->lds_hist = B->lds_conv = B->lds_rw = 0;
+  B->lds_hist = B->lds_conv = B->lds_rw = B->lds_ahead = 0;
+  B->ahead = true;
   for (int i = 0; i < n; ++i) {
     EngineArgs a;
     int rc = engine_args_for(&engines[i], &a);
@@ -284,6 +363,14 @@ extern "C" int phx_batch_create(const phx_engine *engines, int32_t n, void *desc
       delete B;
       return phx::fail(PHX_E_INVALID, "phx_batch_create: engine %d differs from engine 0 in "
                        "record_stats, program_shape or det_shape", i);
+    }
+    B->ahead = B->ahead && a.nsub > 0;
+    if (a.nsub > 0) {
+      const int hb = hist_blocks(e.n);
+      a.hblk = (a.grid + PHX_BATCH_NSUB - 1) / PHX_BATCH_NSUB;
+      a.hblk = a.hblk < hb ? a.hblk : hb;
+      const size_t la = ahead_lds_bytes(e, PHX_BATCH_NSUB);
+      B->lds_ahead = la > B->lds_ahead ? la : B->lds_ahead;
     }
     args[i] = a;
     int nb[BS_COUNT];
@@ -329,9 +416,7 @@ extern "C" int phx_batch_turns(void *batch, int32_t n_turns, phx_stream_t stream
 extern "C" int phx_batch_snapshot(void *batch, phx_stream_t stream) {
   if (!batch) return phx::fail(PHX_E_INVALID, "phx_batch_snapshot: null batch");
   const Batch &B = *reinterpret_cast<Batch *>(batch);
-  k_batch_snapshot<<<dim3(B.n), 64, 0, phx::as_stream(stream)>>>(B.args());
-  PHX_CHECK_LAUNCH("phx_batch_snapshot");
-  return PHX_OK;
+  return batch_begin(B, B.ahead, phx::as_stream(stream));
 }
 
 extern "C" int phx_batch_capture(void *batch, int32_t n_turns, void **graph) {
