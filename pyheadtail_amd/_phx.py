@@ -288,6 +288,11 @@ def check_layouts(lib=None):
 def lib():
     """The library, initialised on the current torch device.  Raises if the
     library or a HIP device is missing: there is no CPU fallback."""
+    # a device that is initialised here is available: is_available() reads the
+    # environment and the driver every time (about 6 us, 10 to 20 calls a turn
+    # in an element loop)
+    if _initialized and torch.cuda.current_device() in _initialized:
+        return _lib
     L = load_library()
     if not torch.cuda.is_available():
         raise PhxError("pyheadtail_amd needs a HIP device: torch.cuda.is_available() is False")
@@ -310,8 +315,9 @@ def call(fn, *args):
 
 
 def stream():
-    """Handle of torch's current HIP stream."""
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of torch's current HIP stream (the handle alone: a torch Stream
+    object costs several us to make)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t):
@@ -346,7 +352,7 @@ class Workspace:
 
     @classmethod
     def get(cls, nbytes):
-        key = (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+        key = (torch.cuda.current_device(), stream())
         buf = cls._cache.get(key)
         if buf is None or buf.numel() < nbytes:
             nb = max(int(nbytes), 1 << 20)
