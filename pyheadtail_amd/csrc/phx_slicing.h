@@ -167,17 +167,6 @@ __device__ __forceinline__ FxScale term_scale(const AccTerms &t, int i, const do
   return fx_scale(bound, n);
 }
 
-__device__ __forceinline__ double term_value(const AccTerms &t, int i, int s, const P6 &p) {
-  double u = p6_get(p, t.a[i]);
-  if (t.ca[i]) u = u - t.ca[i][s];
-  if (t.b[i] >= 0) {
-    double w = p6_get(p, t.b[i]);
-    if (t.cb[i]) w = w - t.cb[i][s];
-    u = u * w;
-  }
-  return u;
-}
-
 // Adds u to sum i of slice s (every call adds one FX_MAGIC to both limbs).  A
 // value beyond the scale's range leaves its nearest multiple of lim in the
 // FP64 fallback (sums of such multiples are exact, so their order does not
@@ -196,13 +185,6 @@ __device__ __forceinline__ void acc_add_value(const AccLds &L, int S, int i, int
   const double l = fma(r, (double)(1LL << FX_LB), FX_MAGIC);
   atomicAdd(&L.hi[(size_t)i * S + s], (unsigned long long)__double_as_longlong(t));
   atomicAdd(&L.lo[(size_t)i * S + s], (unsigned long long)__double_as_longlong(l));
-}
-
-__device__ __forceinline__ void acc_add_lds(const AccLds &L, int S, const AccTerms &t,
-                                            const FxScale *f, int s, const P6 &p,
-                                            double *fallback) {
-  atomicAdd(&L.counts[s], 1u);
-  for (int i = 0; i < t.n; ++i) acc_add_value(L, S, i, s, term_value(t, i, s, p), f[i], fallback);
 }
 
 // Store this block's LDS histogram as partial number h (every entry, zeros

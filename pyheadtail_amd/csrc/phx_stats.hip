@@ -193,45 +193,82 @@ __global__ void k_fill_zero(unsigned long long *p, size_t words) {
 }
 
 #define ACC_BLOCKS 256
+#define ACC_THREADS 1024
 
-__global__ void __launch_bounds__(PHX_BLOCK)
-    k_slice_accumulate(Coords6 co, int64_t n, const phx_slice_state *state, int S, AccTerms terms,
-                       const int32_t *idx_in, int32_t *idx_out, AccParts P) {
+// The distinct centre arrays of the terms (at most two per term), staged in
+// LDS: a centred term otherwise gathers its slices' centres from global
+// memory, up to two gathers of 64 lanes per term and wave.  ia, ib: the
+// staged array of each term's centre_a, centre_b (-1: none).  n = 0: not
+// staged, the centres do not fit beside the sums.
+struct AccCentres {
+  int n;
+  int ia[PHX_MAX_TERMS], ib[PHX_MAX_TERMS];
+  const double *c[2 * PHX_MAX_TERMS];
+};
+
+struct AccItem {
+  int s;
+  P6 p;
+};
+
+// used: bit i, coordinate i is loaded.
+__device__ __forceinline__ AccItem acc_item(const Coords6 &co, unsigned used, int64_t j,
+                                            const int32_t *idx_in, double tail, double width) {
+  AccItem it;
+  it.p.x = used & 1u ? co.c[0][j] : 0.0;
+  it.p.xp = used & 2u ? co.c[1][j] : 0.0;
+  it.p.y = used & 4u ? co.c[2][j] : 0.0;
+  it.p.yp = used & 8u ? co.c[3][j] : 0.0;
+  it.p.z = used & 16u ? co.c[4][j] : 0.0;
+  it.p.dp = used & 32u ? co.c[5][j] : 0.0;
+  it.s = idx_in ? idx_in[j] : x86_cvt_i32(slice_floor(it.p.z, tail, width));
+  return it;
+}
+
+// Bound by the LDS atomics (two 64-bit adds per term and particle) where
+// enough waves hide the loads, so one block fills a CU: NT threads, a particle
+// each and the next one's loads in flight (the sums take most of the LDS, so
+// more blocks would not fit beside it).  T is compiled in: the terms' records
+// stay in scalar registers and the atomics of a particle are independent.
+template <int T, int NT>
+__global__ void __launch_bounds__(NT)
+    k_slice_accumulate(Coords6 co, unsigned used, int64_t n, const phx_slice_state *state, int S,
+                       AccTerms terms, AccCentres cen, const int32_t *idx_in, int32_t *idx_out,
+                       AccParts P) {
   extern __shared__ unsigned long long acc_lds[];
   const double tail = state->tail, width = state->width;
-  __shared__ FxScale f[PHX_MAX_TERMS];
-  if (threadIdx.x < terms.n) f[threadIdx.x] = term_scale(terms, threadIdx.x, state->absmax, n);
-  AccLds L = acc_lds_layout(acc_lds, S, terms.n);
-  acc_lds_zero(L, S, terms.n);
-  const int64_t n_chunks = (n + PHX_CHUNK - 1) / PHX_CHUNK;
-  for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
-    const int64_t base = c * PHX_CHUNK;
+  __shared__ FxScale f[T > 0 ? T : 1];
+  if (threadIdx.x < T) f[threadIdx.x] = term_scale(terms, threadIdx.x, state->absmax, n);
+  AccLds L = acc_lds_layout(acc_lds, S, T);
+  double *ct = reinterpret_cast<double *>(acc_lds + (acc_lds_bytes(S, T) + 7) / 8);
+  for (int k = 0; k < cen.n; ++k)
+    for (int i = threadIdx.x; i < S; i += NT) ct[(size_t)k * S + i] = cen.c[k][i];
+  acc_lds_zero(L, S, T);
+  const int64_t step = (int64_t)gridDim.x * NT;
+  int64_t j = (int64_t)blockIdx.x * NT + threadIdx.x;
+  AccItem cur = {0, {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}}, nxt = cur;
+  if (j < n) cur = acc_item(co, used, j, idx_in, tail, width);
+  for (; j < n; j += step) {
+    if (j + step < n) nxt = acc_item(co, used, j + step, idx_in, tail, width);
+    const int s = cur.s;
+    if (idx_out) idx_out[j] = s;
+    if (s >= 0 && s < S) {
+      atomicAdd(&L.counts[s], 1u);
 #pragma unroll
-    for (int k = 0; k < PHX_PPT; ++k) {
-      const int64_t j = base + (int64_t)k * PHX_BLOCK + threadIdx.x;
-      if (j < n) {
-        const double z = co.c[4] ? co.c[4][j] : 0.0;
-        int s;
-        if (idx_in) {
-          s = idx_in[j];
-        } else {
-          s = x86_cvt_i32(slice_floor(z, tail, width));
+      for (int i = 0; i < T; ++i) {
+        double u = p6_get(cur.p, terms.a[i]);
+        if (terms.ca[i]) u = u - (cen.n ? ct[(size_t)cen.ia[i] * S + s] : terms.ca[i][s]);
+        if (terms.b[i] >= 0) {
+          double w = p6_get(cur.p, terms.b[i]);
+          if (terms.cb[i]) w = w - (cen.n ? ct[(size_t)cen.ib[i] * S + s] : terms.cb[i][s]);
+          u = u * w;
         }
-        if (idx_out) idx_out[j] = s;
-        if (s >= 0 && s < S) {
-          P6 p;
-          p.x = co.c[0] ? co.c[0][j] : 0.0;
-          p.xp = co.c[1] ? co.c[1][j] : 0.0;
-          p.y = co.c[2] ? co.c[2][j] : 0.0;
-          p.yp = co.c[3] ? co.c[3][j] : 0.0;
-          p.z = z;
-          p.dp = co.c[5] ? co.c[5][j] : 0.0;
-          acc_add_lds(L, S, terms, f, s, p, P.fallback);
-        }
+        acc_add_value(L, S, i, s, u, f[i], P.fallback);
       }
     }
+    cur = nxt;
   }
-  acc_lds_store(L, S, terms.n, P, blockIdx.x);
+  acc_lds_store(L, S, T, P, blockIdx.x);
 }
 
 // Merge the partial histograms: counts, exact sums and means per slice;
@@ -289,7 +326,26 @@ extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
   }
   Coords6 co{};
   for (int i = 0; i < 6; ++i) co.c[i] = coords[i];
+  // the coordinates that the terms read, and z where it gives the index
+  unsigned used = idx_in ? 0u : 1u << 4;
+  AccCentres cen{};
+  auto staged = [&](const double *c) {
+    int k = 0;
+    while (k < cen.n && cen.c[k] != c) ++k;
+    if (k == cen.n) cen.c[cen.n++] = c;
+    return k;
+  };
+  for (int i = 0; i < n_terms; ++i) {
+    used |= 1u << t.a[i] | (t.b[i] >= 0 ? 1u << t.b[i] : 0u);
+    cen.ia[i] = t.ca[i] ? staged(t.ca[i]) : -1;
+    cen.ib[i] = t.b[i] >= 0 && t.cb[i] ? staged(t.cb[i]) : -1;
+  }
   const int32_t S = n_slices;
+  size_t lds = (lds_bytes + 7) / 8 * 8 + (size_t)cen.n * S * 8;
+  if (lds + PHX_MAX_TERMS * sizeof(FxScale) > phx_max_lds_bytes()) {
+    cen.n = 0;
+    lds = lds_bytes;
+  }
   const int64_t nc = phx::n_chunks(n);
   const int H = (int)(nc < ACC_BLOCKS ? nc : ACC_BLOCKS);
   char *base = reinterpret_cast<char *>(ws) + phx::WsLayout::kTicketBytes + acc_partials_bytes(n);
@@ -303,16 +359,30 @@ extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
                   s>>>(reinterpret_cast<unsigned long long *>(P.fallback), fw);
     PHX_CHECK_LAUNCH("phx_slice_accumulate: clear");
   }
-  k_slice_accumulate<<<dim3(H), PHX_BLOCK, lds_bytes, s>>>(co, n, state, S, t, idx_in, idx_out,
-                                                           P);
-  PHX_CHECK_LAUNCH("phx_slice_accumulate");
+  // at most a chunk per block: small blocks spread the particles over more CUs
+  const bool small = nc <= ACC_BLOCKS;
   const dim3 mg((S + RD_SL - 1) / RD_SL);
   switch (n_terms) {
-#define PHX_MG(TT) \
-    case TT: k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means); break;
-    PHX_MG(0) PHX_MG(1) PHX_MG(2) PHX_MG(3) PHX_MG(4) PHX_MG(5) PHX_MG(6) PHX_MG(7)
-    default: k_slice_acc_merge<8><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means);
-#undef PHX_MG
+#define PHX_ACC(TT)                                                                            \
+  if (small)                                                                                   \
+    k_slice_accumulate<TT, PHX_BLOCK>                                                          \
+        <<<dim3(H), PHX_BLOCK, lds, s>>>(co, used, n, state, S, t, cen, idx_in, idx_out, P);   \
+  else                                                                                         \
+    k_slice_accumulate<TT, ACC_THREADS>                                                        \
+        <<<dim3(H), ACC_THREADS, lds, s>>>(co, used, n, state, S, t, cen, idx_in, idx_out, P); \
+  PHX_CHECK_LAUNCH("phx_slice_accumulate");                                                    \
+  k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means);   \
+  break;
+    case 0: PHX_ACC(0)
+    case 1: PHX_ACC(1)
+    case 2: PHX_ACC(2)
+    case 3: PHX_ACC(3)
+    case 4: PHX_ACC(4)
+    case 5: PHX_ACC(5)
+    case 6: PHX_ACC(6)
+    case 7: PHX_ACC(7)
+    default: PHX_ACC(8)
+#undef PHX_ACC
   }
   PHX_CHECK_LAUNCH("phx_slice_accumulate: merge");
   return PHX_OK;
