@@ -31,18 +31,22 @@ inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 // What a pass that slices its own turn (ahead_body) needs before it starts,
 // formed by the merge of the turn before it: the turn's cuts, the bounds of
 // x and y that scale its fixed-point sums (those of the state before it),
-// the shift of its z sums (particle 0's z one turn on) and the wake ring's
-// slot and filling after the turn.  One per parity of the turn.
+// the shift of its z sums (particle 0's z one turn on), the wake ring's
+// slot and filling after the turn, the turn and its program.  The merge
+// writes `next` and the convolution copies it to `cur`, which the merge of
+// that turn reads while it writes `next` again: both addresses are known at
+// launch, where a lookup by the turn counter is one or two more dependent
+// loads in kernels of 4 to 8 us.  (The copy is not the pass's: a store ahead
+// of its loop turns its scalar loads into vector loads.)
 struct AheadState {
   double tail, head, width, mean_z, sigma_z, absx, absy, zshift;
-  int nh, nf;
+  int nh, nf, turn, prog;
 };
 
 struct EngineWs {
   double *partials;   // [EN_NV][pass grid] (slot-major)
   double *p0;         // particle 0 before the pass: the shifts of its sums
-  AheadState *ahead;  // [2] (turn parity), in the rest of p0's 256 bytes
-  int *cur_turn;      // the turn of the last such pass
+  AheadState *next, *cur;  // in the rest of p0's 256 bytes
   AccParts acc;       // H partial histograms, T = 2 (x, y)
   double *conv_part;  // [n_kicks][conv_rows(S, T)][S]
 };
@@ -62,9 +66,9 @@ __host__ __device__ inline EngineWs engine_ws(void *ws, int64_t n, int S) {
   w.partials = reinterpret_cast<double *>(p);
   p += ((size_t)nc * EN_NV * 8 + 255) / 256 * 256;
   w.p0 = reinterpret_cast<double *>(p);
-  w.ahead = reinterpret_cast<AheadState *>(p + 64);
-  w.cur_turn = reinterpret_cast<int *>(p + 64 + 2 * sizeof(AheadState));
-  static_assert(64 + 2 * sizeof(AheadState) + sizeof(int) <= 256, "p0 region");
+  w.next = reinterpret_cast<AheadState *>(p + 64);
+  w.cur = w.next + 1;
+  static_assert(64 + 2 * sizeof(AheadState) <= 256, "p0 region");
   p += 256;
   const int H = hist_blocks(n);
   w.acc = acc_parts_layout(p, H, Se, 2);
@@ -317,6 +321,14 @@ __device__ __forceinline__ void group_load(const GroupPtr &gb, uint32_t goff, in
   }
 }
 
+// Byte offset and particle count of group gg (uniform).
+__device__ __forceinline__ int group_at(int64_t gg, int64_t n, uint32_t &off) {
+  const int64_t b = gg * PHX_CHUNK;
+  off = (uint32_t)b * 8u;
+  const int64_t rest = n - b;
+  return rest >= PHX_CHUNK ? PHX_CHUNK : (int)rest;
+}
+
 __device__ __forceinline__ void group_store(const GroupPtr &gb, uint32_t goff, int lim, int tid,
                                             const P6 (&p)[PHX_PPT]) {
 #pragma unroll
@@ -417,9 +429,14 @@ __device__ __forceinline__ void pass_body(
   const phx_engine &e = a.e;
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
   const int64_t n = e.n;
-  const int turn = *e.turn_counter;
-  const int prog_turn = MODE == 0 ? turn : (turn > 0 ? turn - 1 : 0);
-  const phx_turn_program &g = programs[e.turn_program[prog_turn] + stage];
+  int prog;
+  if constexpr (AHEAD) {
+    prog = w.next->prog;
+  } else {
+    const int turn = *e.turn_counter;
+    prog = e.turn_program[MODE == 0 ? turn : (turn > 0 ? turn - 1 : 0)] + stage;
+  }
+  const phx_turn_program &g = programs[prog];
   const int pend = stage == 0 ? *e.pending : 0;
   const int S = e.n_slices;
   const SliceBins bins(e.state->tail, e.state->width, S);
@@ -429,17 +446,10 @@ __device__ __forceinline__ void pass_body(
   const int64_t ng = AHEAD && bid >= nblk ? 0 : phx_n_groups(n);
   // the group's base pointers and particle count (uniform)
   const GroupPtr gb{{x, xp, y, yp, z, dp}};
-  // the group's byte offset and particle count (uniform)
-  auto group = [&](int64_t gg, uint32_t &off) {
-    const int64_t b = gg * PHX_CHUNK;
-    off = (uint32_t)b * 8u;
-    const int64_t rest = n - b;
-    return rest >= PHX_CHUNK ? PHX_CHUNK : (int)rest;
-  };
   int64_t gi = bid;
   uint32_t gc = 0, gnx = 0;
   int lc = 0;
-  if (!AHEAD || gi < ng) lc = group(gi, gc);
+  if (!AHEAD || gi < ng) lc = group_at(gi, n, gc);
   P6 cur[PHX_PPT], nxt[PHX_PPT];
   group_load(gb, gc, lc, tid, cur);
   // Particle 0 sets the shifts of the shifted sums (stats.pyx:cov): its
@@ -467,7 +477,7 @@ __device__ __forceinline__ void pass_body(
     if (MODE == 0 && !AHEAD) apply_shape_longitudinal<SHAPE>(q, g);
     src[6] = q.z;
   }
-  if constexpr (AHEAD) src[6] = w.ahead[turn & 1].zshift;
+  if constexpr (AHEAD) src[6] = w.next->zshift;
   double v[L::NV];
 #pragma unroll
   for (int i = 0; i < L::NV; ++i) v[i] = red_ident<L::MINM, L::MAXM>(i);
@@ -483,7 +493,7 @@ __device__ __forceinline__ void pass_body(
     const int64_t gn = gi + nblk;
     int ln = 0;
     if (gn < ng) {
-      ln = group(gn, gnx);
+      ln = group_at(gn, n, gnx);
       group_load(gb, gnx, ln, tid, nxt);
     }
     if (pend) {
@@ -651,24 +661,23 @@ __device__ __forceinline__ void ahead_body(
   AheadCtx c;
   c.kicks = kt;
   c.acc = acc_lds_layout(reinterpret_cast<unsigned long long *>(pass_lds), S, 2);
+  const AheadState &h = *w.next;
   for (int i = threadIdx.x; i < (int)ahead_kick_doubles(S, KS); i += blockDim.x) kt[i] = kicks[i];
   acc_lds_zero(c.acc, S, 2);  // ends with a barrier; the particle loads follow it
-  const int turn = *e.turn_counter;
-  const AheadState &h = w.ahead[turn & 1];
   c.bins = SliceBins(h.tail, h.width, S);
   c.fx = fx_scale(h.absx, e.n);
   c.fy = fx_scale(h.absy, e.n);
   for (int b0 = 0; b0 < a.grid; b0 += nkb * nsub)
     pass_body<0, REC, true, SHAPE, KS, DS, true>(a, x, xp, y, yp, z, dp, programs, kicks,
                                                  b0 + sub * nkb + kb, a.grid, 0, tid, red, &c);
-  if (kb == 0 && threadIdx.x == 0) *w.cur_turn = turn;
   acc_lds_store(c.acc, S, 2, ahead_parts(w, S, a.hblk), kb);
 }
 
 // The cuts of a three-launch turn from folded z sums, the bounds of |x| and
 // |y| and the ring's state after that turn, into its AheadState (one thread).
 __device__ __forceinline__ void ahead_set(AheadState &h, const phx_slicer &cfg, int64_t n,
-                                          const double *res, int nh, int nf) {
+                                          const double *res, int nh, int nf, int turn,
+                                          int prog) {
   phx_slice_state st;
   compute_cuts(cfg, n, res[0], res[1], res[2], res[3], res[4], st);
   h.tail = st.tail;
@@ -680,6 +689,8 @@ __device__ __forceinline__ void ahead_set(AheadState &h, const phx_slicer &cfg, 
   h.absy = res[7];
   h.nh = nh;
   h.nf = nf;
+  h.turn = turn;
+  h.prog = prog;
 }
 
 // Particle 0's z after two turns' longitudinal motion from c: the shift of
@@ -751,12 +762,14 @@ __device__ __forceinline__ void ahead_start_fold(const EngineArgs &a) {
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
   const int turn = *e.turn_counter;
   const phx_turn_program &g = e.programs[e.turn_program[turn]];
-  AheadState &h = w.ahead[turn & 1];
+  AheadState &h = *w.next;
   if (threadIdx.x < 6) w.p0[threadIdx.x] = e.coords[threadIdx.x][0];
   ahead_fold(w.partials, a.grid, res);
   if (threadIdx.x == 0) {
     const int cap = e.hist->capacity, nf = e.hist->n_filled;
-    ahead_set(h, g.slicer, e.n, res, (e.hist->head + 1) % cap, nf + 1 < cap ? nf + 1 : cap);
+    const int nh = (e.hist->head + 1) % cap, nf1 = nf + 1 < cap ? nf + 1 : cap;
+    ahead_set(h, g.slicer, e.n, res, nh, nf1, turn, e.turn_program[turn]);
+    ahead_set(*w.cur, g.slicer, e.n, res, nh, nf1, turn, e.turn_program[turn]);
   } else if (threadIdx.x == PHX_WAVE) {
     h.zshift = ahead_shift(e.coords, g);
   }
@@ -984,18 +997,37 @@ __host__ __device__ inline int merge_blocks(int S, int SL, bool desc, bool ahead
          (ahead ? MA_STATS + (rec ? MA_STATS_BLOCKS : 0) : 0);
 }
 
+// What merge_slice reads besides the totals, loaded before their reduction.
+struct MergeIn {
+  double beta_c, over_x, over_y;
+  double *times, *mom;  // the new history entry
+};
+
+template <int SL>
+__device__ __forceinline__ MergeIn merge_in(const phx_engine &e, const EngineWs &w, int prog,
+                                            int nh, int s) {
+  const int S = e.n_slices;
+  MergeIn in;
+  in.beta_c = e.programs[prog].beta_c;
+  in.times = e.hist->times + (size_t)nh * S;
+  in.mom = e.hist->mom + (size_t)nh * 3 * S;
+  const bool mine = threadIdx.x < SL && s < S;
+  in.over_x = mine ? w.acc.fallback[s] : 0.0;
+  in.over_y = mine ? w.acc.fallback[S + s] : 0.0;
+  return in;
+}
+
 __device__ __forceinline__ void merge_slice(const phx_engine &e, const EngineWs &w, int s,
-                                            const SliceTotals &tot, int turn, double tail,
-                                            double width, double absx, double absy, int nh) {
+                                            const SliceTotals &tot, const MergeIn &in,
+                                            double tail, double width, double absx, double absy) {
   const int S = e.n_slices;
   // bin edges as np.arange(tail, head + 1e-7*width, width)
   e.z_bins[s] = arange_value(tail, width, s);
   if (s == S - 1) e.z_bins[S] = arange_value(tail, width, S);
-  const phx_turn_program &g = e.programs[e.turn_program[turn]];
   const FxScale fx = fx_scale(absx, e.n), fy = fx_scale(absy, e.n);
   const double cnt = (double)tot.count;
-  const double sx = fx_value(tot.hi[0], tot.lo[0], w.acc.fallback[s], fx);
-  const double sy = fx_value(tot.hi[1], tot.lo[1], w.acc.fallback[S + s], fy);
+  const double sx = fx_value(tot.hi[0], tot.lo[0], in.over_x, fx);
+  const double sy = fx_value(tot.hi[1], tot.lo[1], in.over_y, fy);
   w.acc.fallback[s] = 0.0;
   w.acc.fallback[S + s] = 0.0;
   const double mx = tot.count ? sx / cnt : 0.0;
@@ -1003,14 +1035,12 @@ __device__ __forceinline__ void merge_slice(const phx_engine &e, const EngineWs 
   e.counts[s] = (int32_t)tot.count;
   e.slice_means[s] = mx;
   e.slice_means[S + s] = my;
-  phx_wake_hist *h = e.hist;
   const double zl = arange_value(tail, width, s), zr = arange_value(tail, width, s + 1);
   const double zc = zl + 0.5 * (zr - zl);
-  h->times[(size_t)nh * S + s] = zc / g.beta_c;
-  double *mm = h->mom + (size_t)nh * 3 * S;
-  mm[s] = cnt;
-  mm[S + s] = cnt * mx;
-  mm[2 * S + s] = cnt * my;
+  in.times[s] = zc / in.beta_c;
+  in.mom[s] = cnt;
+  in.mom[S + s] = cnt * mx;
+  in.mom[2 * S + s] = cnt * my;
 }
 
 template <int SL>
@@ -1029,18 +1059,21 @@ __device__ __forceinline__ void merge_body(const EngineArgs &a, int bid) {
     return;
   }
   if (bid == 0 && threadIdx.x == 0) *e.turn_counter = turn + 1;
+  const int s = bid * SL + threadIdx.x % SL;
+  const MergeIn in = merge_in<SL>(e, w, e.turn_program[turn], e.hist->head, s);
+  const double tail = e.state->tail, width = e.state->width;
+  const double absx = e.state->absmax[0], absy = e.state->absmax[2];
   if (!acc_merge<2, SL>(w.acc, S, tot, bid)) return;
-  merge_slice(e, w, bid * SL + threadIdx.x % SL, tot, turn, e.state->tail, e.state->width,
-              e.state->absmax[0], e.state->absmax[2], e.hist->head);
+  merge_slice(e, w, s, tot, in, tail, width, absx, absy);
 }
 
 // The cuts of the next turn and this turn's published state.
 __device__ __forceinline__ void ahead_cuts_block(const EngineArgs &a, const EngineWs &w,
-                                                 int turn) {
+                                                 const AheadState &h) {
   const phx_engine &e = a.e;
   __shared__ double res[ZB_NV];
-  const phx_turn_program &g = e.programs[e.turn_program[turn]];
-  const AheadState &h = w.ahead[turn & 1];
+  const phx_turn_program &g = e.programs[h.prog];
+  const phx_slicer cfg = g.slicer;
   const int cap = e.hist->capacity;
   ahead_fold(w.partials, a.grid, res);
   if (threadIdx.x == 0) {
@@ -1054,14 +1087,14 @@ __device__ __forceinline__ void ahead_cuts_block(const EngineArgs &a, const Engi
     st.absmax[0] = res[5];
     st.absmax[2] = res[7];
     st.n = e.n;
-    st.n_slices = g.slicer.n_slices;
-    st.turn = turn;
+    st.n_slices = cfg.n_slices;
+    st.turn = h.turn;
     st.valid = 1;
     st.pad = 0;
     *e.state = st;
-    ahead_set(w.ahead[(turn & 1) ^ 1], g.slicer, e.n, res, (h.nh + 1) % cap,
-              h.nf + 1 < cap ? h.nf + 1 : cap);
-    *e.turn_counter = turn + 1;
+    ahead_set(*w.next, cfg, e.n, res, (h.nh + 1) % cap, h.nf + 1 < cap ? h.nf + 1 : cap,
+              h.turn + 1, h.prog);
+    *e.turn_counter = h.turn + 1;
   }
 }
 
@@ -1070,17 +1103,16 @@ __device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
   const phx_engine &e = a.e;
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
   const int S = e.n_slices;
-  const int turn = *w.cur_turn;
-  const AheadState &h = w.ahead[turn & 1];
+  const AheadState h = *w.cur;
   const int nm = (S + SL - 1) / SL;
   if (bid >= nm) {
-    const phx_turn_program &g = e.programs[e.turn_program[turn]];
+    const phx_turn_program &g = e.programs[h.prog];
     const int k = bid - nm;
     if (k == MA_CUTS) {
-      ahead_cuts_block(a, w, turn);
+      ahead_cuts_block(a, w, h);
     } else if (k == MA_SHIFT) {
       if (threadIdx.x < 6) w.p0[threadIdx.x] = e.coords[threadIdx.x][0];
-      if (threadIdx.x == PHX_WAVE) w.ahead[(turn & 1) ^ 1].zshift = ahead_shift(e.coords, g);
+      if (threadIdx.x == PHX_WAVE) w.next->zshift = ahead_shift(e.coords, g);
     } else if (k == MA_RING) {
       // the stored entries age by the turn's increment; the new one (slot
       // h.nh) has age 0 (WakeField.track, impedances/wakes.py:134-142)
@@ -1101,7 +1133,7 @@ __device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
       const int i1 = i0 + per < EN_NV ? i0 + per : EN_NV;
       fold_partials<0ULL, 0ULL>(w.partials, a.grid, i0, i1, st);
       if (threadIdx.x < i1 - i0)
-        e.stats[(size_t)turn * EN_STAT_NV + (i0 - ZB_NV) + threadIdx.x] = st[i0 + threadIdx.x];
+        e.stats[(size_t)h.turn * EN_STAT_NV + (i0 - ZB_NV) + threadIdx.x] = st[i0 + threadIdx.x];
     } else {
       rw_desc_build(e.hist, *reinterpret_cast<const WakeKicks *>(g.kick), a.n_kicks, a.T,
                     engine_rw_desc(w, a.n_kicks, S, a.T), h.nf, h.nh, g.beta);
@@ -1109,8 +1141,10 @@ __device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
     return;
   }
   SliceTotals tot;
+  const int s = bid * SL + threadIdx.x % SL;
+  const MergeIn in = merge_in<SL>(e, w, h.prog, h.nh, s);
   if (!acc_merge<2, SL, MA_THREADS>(ahead_parts(w, S, a.hblk), S, tot, bid)) return;
-  merge_slice(e, w, bid * SL + threadIdx.x % SL, tot, turn, h.tail, h.width, h.absx, h.absy, h.nh);
+  merge_slice(e, w, s, tot, in, h.tail, h.width, h.absx, h.absy);
 }
 
 // Space-charge slicing of the state after stage `stage` (the slicing that
@@ -1288,24 +1322,47 @@ __device__ __forceinline__ void sc_merge_body(const EngineArgs &a, int stage, in
 // slices, 7.2 / 6.3 us at 1000); integer sums, the same results.
 __host__ __device__ inline int merge_sl(int S) { return S <= 512 ? 4 : 8; }
 
+// The first block of a turn's convolution: its kicks are pending, and the next
+// turn's AheadState, complete by now, becomes `cur` (a word per thread, loaded
+// ahead of the block's own work and stored after it).
+struct ConvPublish {
+  static constexpr int NW = sizeof(AheadState) / 8;
+  double v;
+  bool mine;
+  __device__ __forceinline__ void begin(const EngineWs &w, bool first_block) {
+    mine = first_block && threadIdx.x < NW;
+    v = mine ? reinterpret_cast<const double *>(w.next)[threadIdx.x] : 0.0;
+  }
+  __device__ __forceinline__ void end(const phx_engine &e, const EngineWs &w) const {
+    if (!mine) return;
+    reinterpret_cast<double *>(w.cur)[threadIdx.x] = v;
+    if (threadIdx.x == 0) *e.pending = 1;
+  }
+};
+static_assert(sizeof(AheadState) % 8 == 0, "AheadState is copied in words");
+
 // Wake convolution block (tile, ki, t) of the general kernel.
 __device__ __forceinline__ void conv_body(const EngineArgs &a, int tile, int ki, int t) {
   const phx_engine &e = a.e;
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
   const phx_turn_program &g = e.programs[e.turn_program[e.state->turn]];
   const WakeKicks &kk = *reinterpret_cast<const WakeKicks *>(g.kick);
-  if (tile == 0 && ki == 0 && t == 0 && threadIdx.x == 0) *e.pending = 1;
+  ConvPublish pub;
+  pub.begin(w, tile == 0 && ki == 0 && t == 0);
   wake_conv_block(e.hist, kk, e.n_slices, w.conv_part, a.T, e.kicks, a.gmax, tile, ki, t,
                   a.n_kicks);
+  pub.end(e, w);
 }
 
 template <int KM>
 __device__ __forceinline__ void conv_rw_body(const EngineArgs &a, int bid) {
   const phx_engine &e = a.e;
   EngineWs w = engine_ws(e.ws, e.n, e.n_slices);
-  if (bid == 0 && threadIdx.x == 0) *e.pending = 1;
+  ConvPublish pub;
+  pub.begin(w, bid == 0);
   wake_rw_block<KM>(e.hist, engine_rw_desc(w, a.n_kicks, e.n_slices, a.T), a.n_kicks,
                     e.n_slices, w.conv_part, a.T, e.kicks, bid);
+  pub.end(e, w);
 }
 
 __device__ __forceinline__ void conv_reduce_body(const EngineArgs &a, int bid) {

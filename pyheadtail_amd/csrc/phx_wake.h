@@ -272,10 +272,25 @@ __device__ __forceinline__ void wake_conv_block(const phx_wake_hist *h, const Wa
   __shared__ double red[WK_GMAX][WK_THREADS];
   __shared__ double rwp[WK_GMAX][3];
   __shared__ WakeKicks kk;
+  // The ring and this thread's time difference (convolution form) come from
+  // memory while the kick table does: after it they would be two more round
+  // trips in a kernel of four.
+  const int nf = h->n_filled, head = h->head, cap = h->capacity;
+  const int slot = ring_slot(head, t, cap);
+  const double age = h->age[slot];
+  const double *tsrc = h->times + (size_t)slot * S;
+  const double *ttgt = h->times + (size_t)head * S;
+  const int j0 = tile * WK_TILE;
+  const double s_last = tsrc[S - 1] + age, s_first = tsrc[0] + age;
+  const int p0 = j0, p1 = min(j0 + WK_TILE - 1 + S - 1, 2 * S - 2);
+  auto conv_dt = [&](int p) {
+    return p <= S - 1 ? ttgt[p] - s_last : ttgt[p - S + 1] - s_first;
+  };
+  int p = p0 + (int)threadIdx.x;
+  const double dt0 = p <= p1 ? conv_dt(p) : 0.0;
   stage_kicks(table, nk, kk);
   const phx_wake_kick &w = kk.k[ki];
   if (is_rw_dot(w)) return;  // wake_rw_block's
-  const int nf = h->n_filled, head = h->head, cap = h->capacity;
   const int n_turns = nf < w.n_turns_wake ? nf : w.n_turns_wake;
   if (t >= n_turns) return;
   int mem[WK_GMAX];
@@ -288,13 +303,8 @@ __device__ __forceinline__ void wake_conv_block(const phx_wake_hist *h, const Wa
     for (int k = ki + 1; k < nk && nm < gmax; ++k)
       if (same_shape(kk.k[k], w)) mem[nm++] = k;
   }
-  const int j0 = tile * WK_TILE;
   const int jj = threadIdx.x % WK_TILE, g = threadIdx.x / WK_TILE;
   const int j = j0 + jj;
-  const int slot = ring_slot(head, t, cap);
-  const double age = h->age[slot];
-  const double *tsrc = h->times + (size_t)slot * S;
-  const double *ttgt = h->times + (size_t)head * S;
   double acc[WK_GMAX];
 #pragma unroll
   for (int m = 0; m < WK_GMAX; ++m) acc[m] = 0.0;
@@ -325,15 +335,16 @@ __device__ __forceinline__ void wake_conv_block(const phx_wake_hist *h, const Wa
     // (wake_kicks.py:109-116)
     double *abuf = vbuf + (WK_TILE + S - 1);
     const double *a = h->mom + ((size_t)slot * 3 + w.moment) * S;
-    for (int i = threadIdx.x; i < S; i += blockDim.x) abuf[i] = a[i];
-    if (threadIdx.x == 0 && w.fn == PHX_WAKE_RESISTIVE_WALL) rw_prefixes(w, h->beta[slot], rwp[0]);
-    lds_sync();
-    const double s_last = tsrc[S - 1] + age, s_first = tsrc[0] + age;
-    const int p0 = j0, p1 = min(j0 + WK_TILE - 1 + S - 1, 2 * S - 2);
-    for (int p = p0 + threadIdx.x; p <= p1; p += blockDim.x) {
-      const double dt = p <= S - 1 ? ttgt[p] - s_last : ttgt[p - S + 1] - s_first;
-      vbuf[p - p0] = wake_eval(w, dt, rwp[0]);
+    // the moments are in flight across the wake values
+    const double a0 = threadIdx.x < S ? a[threadIdx.x] : 0.0;
+    if (w.fn == PHX_WAKE_RESISTIVE_WALL) {
+      if (threadIdx.x == 0) rw_prefixes(w, h->beta[slot], rwp[0]);
+      lds_sync();
     }
+    if (p <= p1) vbuf[p - p0] = wake_eval(w, dt0, rwp[0]);
+    for (p += blockDim.x; p <= p1; p += blockDim.x) vbuf[p - p0] = wake_eval(w, conv_dt(p), rwp[0]);
+    if (threadIdx.x < S) abuf[threadIdx.x] = a0;
+    for (int i = threadIdx.x + blockDim.x; i < S; i += blockDim.x) abuf[i] = a[i];
     lds_sync();
     if (j < S) {
       for (int m = g; m < S; m += WK_GROUPS) acc[0] = acc[0] + abuf[m] * vbuf[j + S - 1 - m - p0];
