@@ -29,7 +29,9 @@ enum { BS_PASS = 0, BS_CUTS, BS_HIST, BS_MERGE, BS_CONV, BS_RW, BS_RWMF, BS_RED,
 // engine's blocks fill a CU each, so that a CU stores one partial histogram;
 // a batch has many times the blocks that are resident, and blocks of one
 // group leave a CU several that start, compute and reduce at different times
-// (8 bunches of 1e6, 20 turns: 6046 us; two groups 6243, three 7576).
+// (20 turns of 8 bunches of 2e5 to 4e6: 5836 us; two groups 6122, three 5825).
+// Fewer blocks a bunch, shared out by its particles, store fewer partial
+// histograms but end less evenly: 0.93 to 1.04 of the time over four scans.
 #define PHX_BATCH_NSUB 1
 
 struct BatchArgs {
@@ -53,11 +55,38 @@ __device__ __forceinline__ int batch_find(const BatchArgs &ba, int stage, int bl
   return lo;
 }
 
+// The record of engine b as the passes read it.  The pointers are loaded
+// through the constant address space (the host fills the table), which tells
+// the compiler that they point to global memory: loaded from plain memory
+// they could point to LDS as well, so every access of the pass was a flat
+// load, and the turn program's values stood in vector registers (214 to 291
+// a thread where the single engine's kernels have 105 to 161).
+__device__ __forceinline__ EngineArgs pass_args(const BatchArgs &ba, int b) {
+  typedef const __attribute__((address_space(4))) EngineArgs ConstArgs;
+  ConstArgs *q = (ConstArgs *)(ba.args + b);
+  EngineArgs a{};
+  for (int i = 0; i < 6; ++i) a.e.coords[i] = q->e.coords[i];
+  a.e.n = q->e.n;
+  a.e.n_slices = q->e.n_slices;
+  a.e.kick_shape = q->e.kick_shape;
+  a.e.programs = q->e.programs;
+  a.e.turn_program = q->e.turn_program;
+  a.e.turn_counter = q->e.turn_counter;
+  a.e.pending = q->e.pending;
+  a.e.state = q->e.state;
+  a.e.kicks = q->e.kicks;
+  a.e.ws = q->e.ws;
+  a.n_kicks = q->n_kicks;
+  a.grid = q->grid;
+  a.hblk = q->hblk;
+  return a;
+}
+
 template <bool REC, int SHAPE, int DS>
 __global__ void __launch_bounds__(PHX_BLOCK) k_batch_pass(BatchArgs ba) {
   int loc;
   const int b = batch_find(ba, BS_PASS, blockIdx.x, loc);
-  const EngineArgs &a = ba.args[b];
+  const EngineArgs a = pass_args(ba, b);
   const phx_engine &e = a.e;
   double *const *c = e.coords;
   if (e.kick_shape == PHX_KICKS_DXDY)
@@ -71,24 +100,56 @@ __global__ void __launch_bounds__(PHX_BLOCK) k_batch_pass(BatchArgs ba) {
                                                           e.programs, e.kicks, loc, a.grid);
 }
 
-// The turn's map and the slicing of every engine.  Bound by its FP64
-// instructions (8 bunches of 1e6: 225 us, about 195 of them); the pass,
-// cuts and histogram launches that it replaces took 205 + 7 + 73 us.  The
-// compiler's own 180..300 registers (two blocks a CU) are the best choice:
-// forced to three blocks it spills (scan of 20 turns 9089 us against 6046).
-template <bool REC, int SHAPE, int DS>
-__global__ void __launch_bounds__(PHX_BLOCK) k_batch_ahead(BatchArgs ba) {
-  int loc;
-  const int b = batch_find(ba, BS_APASS, blockIdx.x, loc);
-  const EngineArgs &a = ba.args[b];
+// A record of read-only memory (uniform address), copied word by word through
+// the constant address space: its words become scalar loads.
+template <class T>
+__device__ __forceinline__ void copy_const(T &dst, const T &src) {
+  static_assert(sizeof(T) % 8 == 0, "whole words");
+  typedef const __attribute__((address_space(4))) uint64_t Word;
+  Word *s = (Word *)&src;
+  uint64_t *d = reinterpret_cast<uint64_t *>(&dst);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(T) / 8); ++i) d[i] = s[i];
+}
+
+template <bool REC, int SHAPE, int KS, int DS>
+__device__ __forceinline__ void batch_ahead(const EngineArgs &a, int loc) {
   const phx_engine &e = a.e;
   double *const *c = e.coords;
-  if (e.kick_shape == PHX_KICKS_DXDY)
-    ahead_body<REC, SHAPE, PHX_KICKS_DXDY, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5], e.programs,
-                                               e.kicks, loc, a.hblk, PHX_BATCH_NSUB);
-  else
-    ahead_body<REC, SHAPE, PHX_KICKS_PLATES, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5],
-                                                 e.programs, e.kicks, loc, a.hblk, PHX_BATCH_NSUB);
+  if constexpr (SHAPE != PHX_SHAPE_GENERIC && DS != PHX_DETS_GENERIC) {
+    // What a compiled element order reads of the turn's program, in scalar
+    // registers: the pass's arguments come from a table, not from the launch,
+    // so the compiler cannot tell the program from the coordinates that the
+    // pass writes, and would load it into vector registers.
+    AheadState h;
+    copy_const(h, *engine_ws(e.ws, e.n, e.n_slices).next);
+    const phx_turn_program &src = e.programs[h.prog];
+    phx_turn_program g;
+    copy_const(g.tseg[0], src.tseg[0]);
+    copy_const(g.lseq[0], src.lseq[0]);
+    copy_const(g.lin[0], src.lin[0]);
+    copy_const(g.slicer, src.slicer);
+    g.has_sc = 0;
+    g.n_kicks = a.n_kicks;
+    ahead_body<REC, SHAPE, KS, DS, AHEAD_OWN>(a, c[0], c[1], c[2], c[3], c[4], c[5], &g, e.kicks,
+                                              loc, a.hblk, PHX_BATCH_NSUB);
+  } else {
+    ahead_body<REC, SHAPE, KS, DS>(a, c[0], c[1], c[2], c[3], c[4], c[5], e.programs, e.kicks,
+                                   loc, a.hblk, PHX_BATCH_NSUB);
+  }
+}
+
+// The turn's map and the slicing of every engine.  Bound by memory with the
+// partial histograms counted (8 bunches, 10.8e6 macroparticles: 215 us for
+// 1.04 GB of coordinates and about 0.1 GB of histograms); 221 us with the
+// program in vector registers (198 a thread instead of 149).
+template <bool REC, int SHAPE, int DS>
+__global__ void __launch_bounds__(PHX_BATCH_NSUB * PHX_BLOCK) k_batch_ahead(BatchArgs ba) {
+  int loc;
+  const int b = batch_find(ba, BS_APASS, blockIdx.x, loc);
+  const EngineArgs a = pass_args(ba, b);
+  if (a.e.kick_shape == PHX_KICKS_DXDY) batch_ahead<REC, SHAPE, PHX_KICKS_DXDY, DS>(a, loc);
+  else batch_ahead<REC, SHAPE, PHX_KICKS_PLATES, DS>(a, loc);
 }
 
 __global__ void __launch_bounds__(PHX_BLOCK) k_batch_ahead_start(BatchArgs ba) {

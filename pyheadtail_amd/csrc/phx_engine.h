@@ -396,6 +396,7 @@ struct PassLayout {
 // are added to the block's slice histogram `acc`, and the z sums are those of
 // the next turn (aheadz: the cuts and scales of ahead_body; bid >= nblk: a
 // group without particles).
+enum { AHEAD_NONE = 0, AHEAD_TABLE, AHEAD_OWN };  // AHEAD_OWN: programs is the turn's program
 struct AheadCtx {
   AccLds acc;
   const double *kicks;  // the pending kick table in LDS
@@ -417,7 +418,7 @@ __device__ __forceinline__ void kick_from_lds(P6 &p, int s, int S, const double 
   }
 }
 
-template <int MODE, bool REC, bool WAKE, int SHAPE, int KS, int DS, bool AHEAD>
+template <int MODE, bool REC, bool WAKE, int SHAPE, int KS, int DS, int AHEAD>
 __device__ __forceinline__ void pass_body(
     const EngineArgs &a, double *__restrict__ x, double *__restrict__ xp,
     double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
@@ -431,7 +432,7 @@ __device__ __forceinline__ void pass_body(
   const int64_t n = e.n;
   int prog;
   if constexpr (AHEAD) {
-    prog = w.next->prog;
+    prog = AHEAD == AHEAD_OWN ? 0 : w.next->prog;
   } else {
     const int turn = *e.turn_counter;
     prog = e.turn_program[MODE == 0 ? turn : (turn > 0 ? turn - 1 : 0)] + stage;
@@ -594,7 +595,7 @@ __device__ __forceinline__ void pass_body(
     double *__restrict__ dp, const phx_turn_program *__restrict__ programs,
     const double *__restrict__ kicks, int bid, int nblk, int stage = 0) {
   extern __shared__ double pass_lds[];
-  pass_body<MODE, REC, WAKE, SHAPE, KS, DS, false>(a, x, xp, y, yp, z, dp, programs, kicks, bid,
+  pass_body<MODE, REC, WAKE, SHAPE, KS, DS, AHEAD_NONE>(a, x, xp, y, yp, z, dp, programs, kicks, bid,
                                                    nblk, stage, threadIdx.x, pass_lds, nullptr);
 }
 
@@ -644,7 +645,7 @@ __device__ __forceinline__ AccParts ahead_parts(const EngineWs &w, int S, int hb
 }
 
 // Pass block kb of nkb.
-template <bool REC, int SHAPE, int KS, int DS>
+template <bool REC, int SHAPE, int KS, int DS, int AHEAD = AHEAD_TABLE>
 __device__ __forceinline__ void ahead_body(
     const EngineArgs &a, double *__restrict__ x, double *__restrict__ xp,
     double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
@@ -668,7 +669,7 @@ __device__ __forceinline__ void ahead_body(
   c.fx = fx_scale(h.absx, e.n);
   c.fy = fx_scale(h.absy, e.n);
   for (int b0 = 0; b0 < a.grid; b0 += nkb * nsub)
-    pass_body<0, REC, true, SHAPE, KS, DS, true>(a, x, xp, y, yp, z, dp, programs, kicks,
+    pass_body<0, REC, true, SHAPE, KS, DS, AHEAD>(a, x, xp, y, yp, z, dp, programs, kicks,
                                                  b0 + sub * nkb + kb, a.grid, 0, tid, red, &c);
   acc_lds_store(c.acc, S, 2, ahead_parts(w, S, a.hblk), kb);
 }
