@@ -123,7 +123,8 @@ __device__ __forceinline__ void batch_ahead(const EngineArgs &a, int loc) {
     // pass writes, and would load it into vector registers.
     AheadState h;
     copy_const(h, *engine_ws(e.ws, e.n, e.n_slices).next);
-    const phx_turn_program &src = e.programs[h.prog];
+    typedef const __attribute__((address_space(4))) int ConstInt;
+    const phx_turn_program &src = e.programs[((ConstInt *)e.turn_program)[h.turn]];
     phx_turn_program g;
     copy_const(g.tseg[0], src.tseg[0]);
     copy_const(g.lseq[0], src.lseq[0]);

@@ -32,15 +32,16 @@ inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 // formed by the merge of the turn before it: the turn's cuts, the bounds of
 // x and y that scale its fixed-point sums (those of the state before it),
 // the shift of its z sums (particle 0's z one turn on), the wake ring's
-// slot and filling after the turn, the turn and its program.  The merge
-// writes `next` and the convolution copies it to `cur`, which the merge of
-// that turn reads while it writes `next` again: both addresses are known at
-// launch, where a lookup by the turn counter is one or two more dependent
-// loads in kernels of 4 to 8 us.  (The copy is not the pass's: a store ahead
+// slot and filling after the turn, and the turn.  The merge writes `next` and
+// the convolution copies it to `cur`, which the merge of that turn reads while
+// it writes `next` again: both addresses are known at launch, where a lookup
+// by the turn counter is one more dependent load in kernels of 4 to 8 us.
+// The program is looked up by the turn: a sequence's first turns may have
+// others whose parameters differ in the last bit.  (The copy is not the pass's: a store ahead
 // of its loop turns its scalar loads into vector loads.)
 struct AheadState {
   double tail, head, width, mean_z, sigma_z, absx, absy, zshift;
-  int nh, nf, turn, prog;
+  int nh, nf, turn, pad;
 };
 
 struct EngineWs {
@@ -432,7 +433,7 @@ __device__ __forceinline__ void pass_body(
   const int64_t n = e.n;
   int prog;
   if constexpr (AHEAD) {
-    prog = AHEAD == AHEAD_OWN ? 0 : w.next->prog;
+    prog = AHEAD == AHEAD_OWN ? 0 : e.turn_program[w.next->turn];
   } else {
     const int turn = *e.turn_counter;
     prog = e.turn_program[MODE == 0 ? turn : (turn > 0 ? turn - 1 : 0)] + stage;
@@ -677,8 +678,7 @@ __device__ __forceinline__ void ahead_body(
 // The cuts of a three-launch turn from folded z sums, the bounds of |x| and
 // |y| and the ring's state after that turn, into its AheadState (one thread).
 __device__ __forceinline__ void ahead_set(AheadState &h, const phx_slicer &cfg, int64_t n,
-                                          const double *res, int nh, int nf, int turn,
-                                          int prog) {
+                                          const double *res, int nh, int nf, int turn) {
   phx_slice_state st;
   compute_cuts(cfg, n, res[0], res[1], res[2], res[3], res[4], st);
   h.tail = st.tail;
@@ -691,7 +691,7 @@ __device__ __forceinline__ void ahead_set(AheadState &h, const phx_slicer &cfg, 
   h.nh = nh;
   h.nf = nf;
   h.turn = turn;
-  h.prog = prog;
+  h.pad = 0;
 }
 
 // Particle 0's z after two turns' longitudinal motion from c: the shift of
@@ -769,8 +769,8 @@ __device__ __forceinline__ void ahead_start_fold(const EngineArgs &a) {
   if (threadIdx.x == 0) {
     const int cap = e.hist->capacity, nf = e.hist->n_filled;
     const int nh = (e.hist->head + 1) % cap, nf1 = nf + 1 < cap ? nf + 1 : cap;
-    ahead_set(h, g.slicer, e.n, res, nh, nf1, turn, e.turn_program[turn]);
-    ahead_set(*w.cur, g.slicer, e.n, res, nh, nf1, turn, e.turn_program[turn]);
+    ahead_set(h, g.slicer, e.n, res, nh, nf1, turn);
+    ahead_set(*w.cur, g.slicer, e.n, res, nh, nf1, turn);
   } else if (threadIdx.x == PHX_WAVE) {
     h.zshift = ahead_shift(e.coords, g);
   }
@@ -1073,7 +1073,7 @@ __device__ __forceinline__ void ahead_cuts_block(const EngineArgs &a, const Engi
                                                  const AheadState &h) {
   const phx_engine &e = a.e;
   __shared__ double res[ZB_NV];
-  const phx_turn_program &g = e.programs[h.prog];
+  const phx_turn_program &g = e.programs[e.turn_program[h.turn]];
   const phx_slicer cfg = g.slicer;
   const int cap = e.hist->capacity;
   ahead_fold(w.partials, a.grid, res);
@@ -1094,7 +1094,7 @@ __device__ __forceinline__ void ahead_cuts_block(const EngineArgs &a, const Engi
     st.pad = 0;
     *e.state = st;
     ahead_set(*w.next, cfg, e.n, res, (h.nh + 1) % cap, h.nf + 1 < cap ? h.nf + 1 : cap,
-              h.turn + 1, h.prog);
+              h.turn + 1);
     *e.turn_counter = h.turn + 1;
   }
 }
@@ -1107,7 +1107,7 @@ __device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
   const AheadState h = *w.cur;
   const int nm = (S + SL - 1) / SL;
   if (bid >= nm) {
-    const phx_turn_program &g = e.programs[h.prog];
+    const phx_turn_program &g = e.programs[e.turn_program[h.turn]];
     const int k = bid - nm;
     if (k == MA_CUTS) {
       ahead_cuts_block(a, w, h);
@@ -1143,7 +1143,7 @@ __device__ __forceinline__ void ahead_merge_body(const EngineArgs &a, int bid) {
   }
   SliceTotals tot;
   const int s = bid * SL + threadIdx.x % SL;
-  const MergeIn in = merge_in<SL>(e, w, h.prog, h.nh, s);
+  const MergeIn in = merge_in<SL>(e, w, e.turn_program[h.turn], h.nh, s);
   if (!acc_merge<2, SL, MA_THREADS>(ahead_parts(w, S, a.hblk), S, tot, bid)) return;
   merge_slice(e, w, s, tot, in, h.tail, h.width, h.absx, h.absy);
 }
