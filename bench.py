@@ -251,11 +251,11 @@ def record_traffic(d, n):
     """profiles/pass_traffic.json: the pass's FETCH_SIZE and WRITE_SIZE (KiB
     per dispatch) at n macroparticles and the same counters for a plain copy
     of the six coordinate arrays, with the digest of the sources built."""
-    fetch, nd = _counter_means(os.path.join(d, "fetch_pass"), "FETCH_SIZE", "k_engine_pass")
-    write, _ = _counter_means(os.path.join(d, "write_pass"), "WRITE_SIZE", "k_engine_pass")
+    fetch, nd = _counter_means(os.path.join(d, "fetch_pass"), "FETCH_SIZE", "k_engine_ahead<")
+    write, _ = _counter_means(os.path.join(d, "write_pass"), "WRITE_SIZE", "k_engine_ahead<")
     cfetch, _ = _counter_means(os.path.join(d, "fetch_copy"), "FETCH_SIZE", "opy")
     cwrite, _ = _counter_means(os.path.join(d, "write_copy"), "WRITE_SIZE", "opy")
-    rec = {"kernel": "k_engine_pass (headline map)", "macroparticles": n,
+    rec = {"kernel": "k_engine_ahead (headline map)", "macroparticles": n,
            "fetch_kib": fetch, "write_kib": write, "dispatches": nd,
            "copy_bytes": 48 * n, "copy_fetch_kib": cfetch, "copy_write_kib": cwrite,
            "sources_sha256": sources_sha256()}
@@ -779,7 +779,7 @@ def main():
                                % (args.n, args.slices),
                    "macroparticles": args.n, "n_slices": args.slices, "turns": args.steps,
                    "graph_turns": args.graph_turns},
-        "roofline": roofline(args.n, stage_ms[0], "k_engine_pass (fused particle pass)"),
+        "roofline": roofline(args.n, stage_ms[0], "k_engine_ahead (particle pass with slicing)"),
         "turn_roofline_frac": BYTES_PER_MP_PASS * args.n / (turn_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
         "stage_ms": {"pass": stage_ms[0], "hist": stage_ms[1], "conv": stage_ms[2]},
         "h2d_bunch_ms": h2d_ms,
@@ -794,7 +794,7 @@ def main():
             "macroparticles": args.n_large, "turns": steps_l,
             "value": args.n_large * steps_l / dt_l, "ms_per_step": dt_l / steps_l * 1e3,
             "stage_ms": {"pass": st_l[0], "hist": st_l[1], "conv": st_l[2]},
-            "roofline": roofline(args.n_large, st_l[0], "k_engine_pass (fused particle pass)"),
+            "roofline": roofline(args.n_large, st_l[0], "k_engine_ahead (particle pass with slicing)"),
             "turn_roofline_frac": (BYTES_PER_MP_PASS * args.n_large / (dt_l / steps_l) / 1e9 /
                                    HBM_PEAK_GBS),
         }
