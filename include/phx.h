@@ -179,6 +179,23 @@ int phx_slice_accumulate(const double *const coords[6], int64_t n,
                          double *sums, double *means,
                          void *ws, phx_stream_t stream);
 
+/*
+ * phx_slice_accumulate with the sums of the slice statistics: every value is
+ * kept to the fixed quantum 2^(ilogb(bound) - 60), bound being the term's from
+ * max|u| (phx_slice_accumulate: finer, 2^-64 of the bound or less).  The
+ * covariance of a slice of two or three macroparticles is singular, so that
+ * its emittance (phx_slice_finalize, kind 2) is the root of what the sums
+ * round to: which of these slices give NaN, and the others' values, depend on
+ * the quantum, which therefore stays.
+ */
+int phx_slice_moments(const double *const coords[6], int64_t n,
+                      const phx_slice_state *state, int32_t n_slices,
+                      const phx_term *terms, int32_t n_terms,
+                      const int32_t *idx_in, int32_t *idx_out,
+                      int32_t *counts,
+                      double *sums, double *means,
+                      void *ws, phx_stream_t stream);
+
 /* Per-slice statistics from centred second-moment sums (device arrays of
  * length n_slices):  kind 0: std  = sqrt(c_aa/(n-1))        (stats.pyx:258-286)
  *                    kind 1: cov  = c_ab/(n-1)              (stats.pyx:290-319)

@@ -217,6 +217,7 @@ SIGNATURES = {
     "phx_bunch_sums": (C.c_int, [P, I32, I64, P, P, P]),
     "phx_slice_cuts": (C.c_int, [P, I64, P, P, P, P, P]),
     "phx_slice_accumulate": (C.c_int, [P, I64, P, I32, P, I32, P, P, P, P, P, P, P]),
+    "phx_slice_moments": (C.c_int, [P, I64, P, I32, P, I32, P, P, P, P, P, P, P]),
     "phx_slice_finalize": (C.c_int, [I32, I32, P, P, I32, D, D, D, P, P]),
     "phx_slice_times": (C.c_int, [P, I32, D, P, P, P]),
     "phx_transverse_segment": (C.c_int, [P, P, P, P, P, I64, P, P]),

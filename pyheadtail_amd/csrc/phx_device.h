@@ -737,6 +737,37 @@ __device__ __forceinline__ double fx_value(unsigned long long hi_sum, unsigned l
   return in ? v : v + over;
 }
 
+// The scale of the slice statistics (phx_slice_moments): every value is kept
+// to the fixed quantum 2^(ilogb(bound) - 60), the integer h 2^FX_LB + l.  The
+// covariance of a slice of two or three macroparticles is singular, its
+// emittance the root of what the sums round to (a small number, or NaN), so
+// the quantum is part of the result.  Terms up to 2^(ilogb(bound) + 2) stay
+// in the limbs; h is below 2^22, its sums below 2^53 for up to 2^31 terms.
+// No scale can be taken from a bound of zero, below 2^-1000 or beyond FX_HUGE
+// (an infinity among the values): fx_scale's then, as its sums.
+__device__ __forceinline__ bool fx_has_quantum(double bound) {
+  return bound >= 0x1p-1000 && bound < FX_HUGE;
+}
+
+__device__ __forceinline__ FxScale fx_scale_quantum(double bound, int64_t n) {
+  if (!fx_has_quantum(bound)) return fx_scale(bound, n);
+  const int il = __builtin_amdgcn_frexp_exp(bound) - 1;
+  return FxScale{fx_pow2(60 - FX_LB - il), fx_pow2(il + 2), fx_pow2(il + FX_LB - 60)};
+}
+
+// The sum of fx_scale_quantum's limbs: the integer, its upper part (from 2^32
+// on) and its lower 32 bits each as a double, added and scaled.
+__device__ __forceinline__ double fx_value_quantum(unsigned long long hi_sum,
+                                                   unsigned long long lo_sum, double over,
+                                                   double bound, const FxScale &f) {
+  if (!fx_has_quantum(bound)) return fx_value(hi_sum, lo_sum, over, f);
+  const long long h = (long long)hi_sum + (long long)(lo_sum >> FX_LB);
+  const unsigned long long l = lo_sum & ((1ULL << FX_LB) - 1ULL);
+  const long long top = h * (1LL << (FX_LB - 32)) + (long long)(l >> 32);
+  const double s = (double)top * 0x1p32 + (double)(l & 0xffffffffULL);
+  return (s * (1.0 / (double)(1LL << FX_LB))) * f.unit + over;
+}
+
 // ---------------------------------------------------------------------------
 // Cuts of UniformBinSlicer (particles/slicing.py:395-413, 599-615) from the
 // reduced z sums, and z_bins as np.arange(tail, head + 1e-7*width, width):

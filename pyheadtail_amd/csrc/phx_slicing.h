@@ -157,14 +157,12 @@ __device__ __forceinline__ void acc_lds_zero(const AccLds &L, int S, int T) {
   lds_sync();
 }
 
-// The scale of a term's sums from max|u| (centres are per-slice means, |c| <=
-// max|u|).
-__device__ __forceinline__ FxScale term_scale(const AccTerms &t, int i, const double *absmax,
-                                              int64_t n) {
+// Bound of |term| from max|u| (centres are per-slice means, |c| <= max|u|).
+__device__ __forceinline__ double term_bound(const AccTerms &t, int i, const double *absmax) {
   double ba = absmax[t.a[i]] * (t.ca[i] ? 2.0 : 1.0);
   double bound = ba;
   if (t.b[i] >= 0) bound = ba * (absmax[t.b[i]] * (t.cb[i] ? 2.0 : 1.0));
-  return fx_scale(bound, n);
+  return bound;
 }
 
 // Adds u to sum i of slice s (every call adds one FX_MAGIC to both limbs).  A

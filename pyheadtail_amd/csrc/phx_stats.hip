@@ -238,12 +238,15 @@ __device__ __forceinline__ AccItem acc_item(const Coords6 &co, unsigned used, in
 template <int T, int NT>
 __global__ void __launch_bounds__(NT)
     k_slice_accumulate(Coords6 co, unsigned used, int64_t n, const phx_slice_state *state, int S,
-                       AccTerms terms, AccCentres cen, const int32_t *idx_in, int32_t *idx_out,
-                       AccParts P) {
+                       AccTerms terms, AccCentres cen, bool quantum, const int32_t *idx_in,
+                       int32_t *idx_out, AccParts P) {
   extern __shared__ unsigned long long acc_lds[];
   const double tail = state->tail, width = state->width;
   __shared__ FxScale f[T > 0 ? T : 1];
-  if (threadIdx.x < T) f[threadIdx.x] = term_scale(terms, threadIdx.x, state->absmax, n);
+  if (threadIdx.x < T) {
+    const double bound = term_bound(terms, threadIdx.x, state->absmax);
+    f[threadIdx.x] = quantum ? fx_scale_quantum(bound, n) : fx_scale(bound, n);
+  }
   AccLds L = acc_lds_layout(acc_lds, S, T);
   double *ct = reinterpret_cast<double *>(acc_lds + (acc_lds_bytes(S, T) + 7) / 8);
   for (int k = 0; k < cen.n; ++k)
@@ -276,12 +279,12 @@ __global__ void __launch_bounds__(NT)
   acc_lds_store(L, S, T, P, blockIdx.x);
 }
 
-// Merge the partial histograms: counts, exact sums and means per slice;
-// re-zero the FP64 fallback entries.
+// Merge the partial histograms: counts, sums and means per slice (quantum: of
+// fx_scale_quantum's integers); re-zero the FP64 fallback entries.
 template <int T>
 __global__ void __launch_bounds__(RD_SL * RD_G)
     k_slice_acc_merge(AccParts P, int S, AccTerms terms, const phx_slice_state *state, int64_t n,
-                      int32_t *counts, double *sums, double *means) {
+                      bool quantum, int32_t *counts, double *sums, double *means) {
   SliceTotals tot;
   if (!acc_merge<T>(P, S, tot, blockIdx.x)) return;
   const int s = blockIdx.x * RD_SL + threadIdx.x % RD_SL;
@@ -289,41 +292,41 @@ __global__ void __launch_bounds__(RD_SL * RD_G)
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     const size_t k = (size_t)i * S + s;
-    const double v = fx_value(tot.hi[i], tot.lo[i], P.fallback[k],
-                              term_scale(terms, i, state->absmax, n));
+    const double bound = term_bound(terms, i, state->absmax);
+    const double v = quantum ? fx_value_quantum(tot.hi[i], tot.lo[i], P.fallback[k], bound,
+                                                fx_scale_quantum(bound, n))
+                             : fx_value(tot.hi[i], tot.lo[i], P.fallback[k], fx_scale(bound, n));
     P.fallback[k] = 0.0;
     if (sums) sums[k] = v;
     if (means) means[k] = tot.count ? v / (double)tot.count : 0.0;
   }
 }
 
-extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
-                                    const phx_slice_state *state, int32_t n_slices,
-                                    const phx_term *terms, int32_t n_terms,
-                                    const int32_t *idx_in, int32_t *idx_out, int32_t *counts,
-                                    double *sums, double *means, void *ws,
-                                    phx_stream_t stream) {
+static int slice_accumulate(const char *who, bool quantum, const double *const coords[6],
+                            int64_t n, const phx_slice_state *state, int32_t n_slices,
+                            const phx_term *terms, int32_t n_terms, const int32_t *idx_in,
+                            int32_t *idx_out, int32_t *counts, double *sums, double *means,
+                            void *ws, phx_stream_t stream) {
   if (!coords || (!coords[4] && !idx_in) || !state || !counts || !ws)
-    return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: null pointer");
-  if (n < 1) return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: n=%lld < 1", (long long)n);
-  if (n_slices < 1) return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: n_slices < 1");
+    return phx::fail(PHX_E_INVALID, "%s: null pointer", who);
+  if (n < 1) return phx::fail(PHX_E_INVALID, "%s: n=%lld < 1", who, (long long)n);
+  if (n_slices < 1) return phx::fail(PHX_E_INVALID, "%s: n_slices < 1", who);
   if (n_terms < 0 || n_terms > PHX_MAX_TERMS)
-    return phx::fail(PHX_E_LIMIT, "phx_slice_accumulate: n_terms=%d not in 0..%d", n_terms,
-                     PHX_MAX_TERMS);
+    return phx::fail(PHX_E_LIMIT, "%s: n_terms=%d not in 0..%d", who, n_terms, PHX_MAX_TERMS);
   if (n_terms > 0 && (!terms || !sums))
-    return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: terms/sums null");
+    return phx::fail(PHX_E_INVALID, "%s: terms/sums null", who);
   const size_t lds_bytes = acc_lds_bytes(n_slices, n_terms);
   if (lds_bytes > phx_max_lds_bytes())
     return phx::fail(PHX_E_LIMIT,
-                     "phx_slice_accumulate: %d slices x %d terms need %zu B of LDS (max %zu)",
-                     n_slices, n_terms, lds_bytes, phx_max_lds_bytes());
+                     "%s: %d slices x %d terms need %zu B of LDS (max %zu)", who, n_slices,
+                     n_terms, lds_bytes, phx_max_lds_bytes());
   AccTerms t{};
   t.n = n_terms;
   for (int i = 0; i < n_terms; ++i) {
     if (terms[i].a < 0 || terms[i].a > 5 || terms[i].b > 5)
-      return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: bad coordinate index in term %d", i);
+      return phx::fail(PHX_E_INVALID, "%s: bad coordinate index in term %d", who, i);
     if (!coords[terms[i].a] || (terms[i].b >= 0 && !coords[terms[i].b]))
-      return phx::fail(PHX_E_INVALID, "phx_slice_accumulate: term %d uses a null coordinate", i);
+      return phx::fail(PHX_E_INVALID, "%s: term %d uses a null coordinate", who, i);
     t.a[i] = terms[i].a;
     t.b[i] = terms[i].b;
     t.ca[i] = terms[i].center_a;
@@ -368,15 +371,16 @@ extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
   const bool small = nc <= ACC_BLOCKS;
   const dim3 mg((S + RD_SL - 1) / RD_SL);
   switch (n_terms) {
-#define PHX_ACC(TT)                                                                            \
-  if (small)                                                                                   \
-    k_slice_accumulate<TT, PHX_BLOCK>                                                          \
-        <<<dim3(H), PHX_BLOCK, lds, s>>>(co, used, n, state, S, t, cen, idx_in, idx_out, P);   \
-  else                                                                                         \
-    k_slice_accumulate<TT, ACC_THREADS>                                                        \
-        <<<dim3(H), ACC_THREADS, lds, s>>>(co, used, n, state, S, t, cen, idx_in, idx_out, P); \
-  PHX_CHECK_LAUNCH("phx_slice_accumulate");                                                    \
-  k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, counts, sums, means);   \
+#define PHX_ACC(TT)                                                                         \
+  if (small)                                                                                \
+    k_slice_accumulate<TT, PHX_BLOCK><<<dim3(H), PHX_BLOCK, lds, s>>>(                      \
+        co, used, n, state, S, t, cen, quantum, idx_in, idx_out, P);                        \
+  else                                                                                      \
+    k_slice_accumulate<TT, ACC_THREADS><<<dim3(H), ACC_THREADS, lds, s>>>(                  \
+        co, used, n, state, S, t, cen, quantum, idx_in, idx_out, P);                        \
+  PHX_CHECK_LAUNCH("phx_slice_accumulate");                                                 \
+  k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, quantum, counts,     \
+                                                    sums, means);                           \
   break;
     case 0: PHX_ACC(0)
     case 1: PHX_ACC(1)
@@ -391,6 +395,25 @@ extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
   }
   PHX_CHECK_LAUNCH("phx_slice_accumulate: merge");
   return PHX_OK;
+}
+
+extern "C" int phx_slice_accumulate(const double *const coords[6], int64_t n,
+                                    const phx_slice_state *state, int32_t n_slices,
+                                    const phx_term *terms, int32_t n_terms,
+                                    const int32_t *idx_in, int32_t *idx_out, int32_t *counts,
+                                    double *sums, double *means, void *ws,
+                                    phx_stream_t stream) {
+  return slice_accumulate("phx_slice_accumulate", false, coords, n, state, n_slices, terms,
+                          n_terms, idx_in, idx_out, counts, sums, means, ws, stream);
+}
+
+extern "C" int phx_slice_moments(const double *const coords[6], int64_t n,
+                                 const phx_slice_state *state, int32_t n_slices,
+                                 const phx_term *terms, int32_t n_terms, const int32_t *idx_in,
+                                 int32_t *idx_out, int32_t *counts, double *sums, double *means,
+                                 void *ws, phx_stream_t stream) {
+  return slice_accumulate("phx_slice_moments", true, coords, n, state, n_slices, terms, n_terms,
+                          idx_in, idx_out, counts, sums, means, ws, stream);
 }
 
 // ---------------------------------------------------------------------------
