@@ -341,7 +341,7 @@ class FusedOneTurnMap(Element):
             table[t] = index[key] * n_st
             t += 1
             if self._state_key(state) == before:
-                table[t:] = index[key]
+                table[t:] = index[key] * n_st
                 break
         state.write_back(beam)
         return progs, table
