@@ -562,8 +562,9 @@ enum {
 /* Flag added to PHX_SHAPE_RF1_T: every program's RF sequence is stationary,
    its drifts with beta_ratio = 1 and its kick with phi_offset = phi_lock =
    p_increment = +0 and no dispersion.  The pass then drops those terms,
-   which leave the values unchanged (1 * z = z, (a + 0) + 0 = a + 0,
-   b - 0 = b): the same bits as the general form. */
+   which leave the values unchanged (1 * z = z, a + 0 = a, b - 0 = b): the
+   same bits as the general form.  The ratio p0_before / p0_after stays: the
+   round trip p0 -> gamma -> p0 of a kick may move p0's last bit. */
 #define PHX_SHAPE_STATIONARY 16
 /* Space-charge kicks per turn of the fused engine. */
 #define PHX_MAX_SC_STAGES 16

@@ -304,7 +304,7 @@ __device__ __forceinline__ void apply_tseg_n(P6 (&p)[N], const phx_tseg &t) {
 // ---------------------------------------------------------------------------
 // STAT: a stationary RF sequence (PHX_SHAPE_STATIONARY): beta_ratio = 1,
 // phi_offset = phi_lock = p_increment = +0 and no dispersion, checked by the
-// host, so that 1 * z = z, a phase offset of +0 and fma(dp, 1, -0) = dp drop
+// host, so that 1 * z = z, a phase offset of +0 and fma(dp, r, -0) = dp r drop
 // those terms with the same bits.
 template <int N, bool STAT = false>
 __device__ __forceinline__ void drift_n(P6 (&p)[N], const phx_long_op &o) {
@@ -328,19 +328,19 @@ __device__ __forceinline__ void rf_kick_n(P6 (&p)[N], const phx_long_op &o) {
   // with phi in turns and the quotients by C and p0_after folded into the
   // kick's constants
   const double hz = o.harmonic * o.inv_circumference, amp = o.amplitude * o.inv_p0_after;
+  const double ratio = o.p0_before == o.p0_after ? 1.0 : o.p0_before / o.p0_after;
   double u[N], sn[N];
   if constexpr (STAT) {
 #pragma unroll
     for (int k = 0; k < N; ++k) u[k] = fma(p[k].z, hz, 0.0);
     phx_sin_turns_n<N>(u, sn);
 #pragma unroll
-    for (int k = 0; k < N; ++k) p[k].dp = fma(amp, sn[k], p[k].dp);
+    for (int k = 0; k < N; ++k) p[k].dp = fma(amp, sn[k], p[k].dp * ratio);
     return;
   }
   const bool disp = o.with_dispersion != 0;
   const double Dx = o.D_x, Dy = o.D_y;
   const double off = (o.phi_offset + o.phi_lock) * (1.0 / phx_math::TWO_PI);
-  const double ratio = o.p0_before == o.p0_after ? 1.0 : o.p0_before / o.p0_after;
   const double pinc = -(o.p_increment * o.inv_p0_after);
 #pragma unroll
   for (int k = 0; k < N; ++k) {
