@@ -235,17 +235,26 @@ __device__ __forceinline__ AccItem acc_item(const Coords6 &co, unsigned used, in
 // each and the next one's loads in flight (the sums take most of the LDS, so
 // more blocks would not fit beside it).  T is compiled in: the terms' records
 // stay in scalar registers and the atomics of a particle are independent.
-template <int T, int NT>
+// FULL: the sums alone fill the LDS (8192 slices with one term, 1241 with
+// eight), which leaves no room for the terms' scales (three doubles a term, too
+// many for registers): they are formed where they are used.
+template <int T, int NT, bool FULL>
 __global__ void __launch_bounds__(NT)
     k_slice_accumulate(Coords6 co, unsigned used, int64_t n, const phx_slice_state *state, int S,
                        AccTerms terms, AccCentres cen, bool quantum, const int32_t *idx_in,
                        int32_t *idx_out, AccParts P) {
   extern __shared__ unsigned long long acc_lds[];
   const double tail = state->tail, width = state->width;
-  __shared__ FxScale f[T > 0 ? T : 1];
-  if (threadIdx.x < T) {
-    const double bound = term_bound(terms, threadIdx.x, state->absmax);
-    f[threadIdx.x] = quantum ? fx_scale_quantum(bound, n) : fx_scale(bound, n);
+  auto scale = [&](int i) {
+    const double bound = term_bound(terms, i, state->absmax);
+    return quantum ? fx_scale_quantum(bound, n) : fx_scale(bound, n);
+  };
+  constexpr bool STAGED = T > 0 && !FULL;
+  FxScale *f = nullptr;
+  if constexpr (STAGED) {
+    __shared__ FxScale staged[T];
+    f = staged;
+    if (threadIdx.x < T) f[threadIdx.x] = scale(threadIdx.x);
   }
   AccLds L = acc_lds_layout(acc_lds, S, T);
   double *ct = reinterpret_cast<double *>(acc_lds + (acc_lds_bytes(S, T) + 7) / 8);
@@ -271,7 +280,8 @@ __global__ void __launch_bounds__(NT)
           if (terms.cb[i]) w = w - (cen.n ? ct[(size_t)cen.ib[i] * S + s] : terms.cb[i][s]);
           u = u * w;
         }
-        acc_add_value(L, S, i, s, u, f[i], P.fallback);
+        if constexpr (STAGED) acc_add_value(L, S, i, s, u, f[i], P.fallback);
+        else acc_add_value(L, S, i, s, u, scale(i), P.fallback);
       }
     }
     cur = nxt;
@@ -350,10 +360,12 @@ static int slice_accumulate(const char *who, bool quantum, const double *const c
   }
   const int32_t S = n_slices;
   size_t lds = (lds_bytes + 7) / 8 * 8 + (size_t)cen.n * S * 8;
-  if (lds + PHX_MAX_TERMS * sizeof(FxScale) > phx_max_lds_bytes()) {
+  const size_t scales = (size_t)n_terms * sizeof(FxScale);
+  if (lds + scales > phx_max_lds_bytes()) {
     cen.n = 0;
     lds = lds_bytes;
   }
+  const bool full = lds + scales > phx_max_lds_bytes();
   const int64_t nc = phx::n_chunks(n);
   const int H = (int)(nc < ACC_BLOCKS ? nc : ACC_BLOCKS);
   char *base = reinterpret_cast<char *>(ws) + phx::WsLayout::kTicketBytes + acc_partials_bytes(n);
@@ -372,11 +384,14 @@ static int slice_accumulate(const char *who, bool quantum, const double *const c
   const dim3 mg((S + RD_SL - 1) / RD_SL);
   switch (n_terms) {
 #define PHX_ACC(TT)                                                                         \
-  if (small)                                                                                \
-    k_slice_accumulate<TT, PHX_BLOCK><<<dim3(H), PHX_BLOCK, lds, s>>>(                      \
+  if (full)                                                                                 \
+    k_slice_accumulate<TT, ACC_THREADS, true><<<dim3(H), ACC_THREADS, lds, s>>>(            \
+        co, used, n, state, S, t, cen, quantum, idx_in, idx_out, P);                        \
+  else if (small)                                                                           \
+    k_slice_accumulate<TT, PHX_BLOCK, false><<<dim3(H), PHX_BLOCK, lds, s>>>(               \
         co, used, n, state, S, t, cen, quantum, idx_in, idx_out, P);                        \
   else                                                                                      \
-    k_slice_accumulate<TT, ACC_THREADS><<<dim3(H), ACC_THREADS, lds, s>>>(                  \
+    k_slice_accumulate<TT, ACC_THREADS, false><<<dim3(H), ACC_THREADS, lds, s>>>(           \
         co, used, n, state, S, t, cen, quantum, idx_in, idx_out, P);                        \
   PHX_CHECK_LAUNCH("phx_slice_accumulate");                                                 \
   k_slice_acc_merge<TT><<<mg, RD_SL * RD_G, 0, s>>>(P, S, t, state, n, quantum, counts,     \
