@@ -26,6 +26,7 @@ MAX_PROGRAM = 16
 MAX_SC_STAGES = 16       # space-charge kicks per turn of the fused engine
 STANDALONE_GRID = 768
 MAX_GRID = 2048
+AHEAD_MIN_TURNS = 4      # PHX_AHEAD_MIN_TURNS
 
 CUTS_FIXED, CUTS_NSIGMA, CUTS_MINMAX = 0, 1, 2
 DET_CHROMA, DET_AMPLITUDE = 1, 2

@@ -485,11 +485,12 @@ class FusedOneTurnMap(Element):
         if not np.array_equal(b['host_table'][:n_turns], table):
             b['table'][:n_turns].copy_(torch.from_numpy(table))
             b['host_table'][:n_turns] = table
-        # the turns before the program settles (an RF kick re-derives p0 from
-        # gamma, which moves its last bit in the first turn) run one by one
+        # the turns before the program settles: an RF kick re-derives p0 from
+        # gamma, which moves its last bit in the first turns of about half of
+        # all rings; all but the last of an accelerating one
         moving = np.flatnonzero(np.diff(table))
         self._unsteady = int(moving[-1]) + 1 if len(moving) else 0
-        eng = self._engine_record(beam, b, self._unsteady < n_turns)
+        eng = self._engine_record(beam, b, n_turns - self._unsteady >= _phx.AHEAD_MIN_TURNS)
         self._engine = eng
         if b.get('needs_reset'):
             _phx.call(L.phx_engine_reset, C.byref(eng), _phx.stream())
@@ -506,26 +507,24 @@ class FusedOneTurnMap(Element):
         elif self.record_stats:
             self._finish_stats(beam)
 
-    def _begin(self, eng, s, n_turns):
+    def _begin(self, eng, s, use_graph):
         """Runs the first turns of a call where they need another launch
         sequence than the rest; returns their number."""
         k = self._unsteady if eng.ahead else 0
         if k:
             eng.ahead = 0
-            _phx.call(_phx.lib().phx_engine_turns, C.byref(eng), k, s)
+            self._advance(eng, s, k, use_graph)
             eng.ahead = 1
         return k
 
-    def track_turns(self, beam, n_turns, use_graph=True):
-        """Advance beam by n_turns turns."""
-        if n_turns <= 0:
-            return
+    def _advance(self, eng, s, n_turns, use_graph):
+        """n_turns turns of one launch sequence: the graph's replays (it looks
+        the programs up by the turn, so it serves changing ones too), then
+        the rest."""
         L = _phx.lib()
-        eng = self._prepare(beam, n_turns)
-        s = _phx.stream()
         G = self.graph_turns
-        done = self._begin(eng, s, n_turns)
-        if use_graph and G > 0 and n_turns - done >= G:
+        done = 0
+        if use_graph and G > 0 and n_turns >= G:
             key = (tuple(eng.coords), self.record_stats, G, self._shape, eng.ahead)
             h = self._graphs.get(key)
             if h is None:
@@ -538,6 +537,15 @@ class FusedOneTurnMap(Element):
                 done += G
         if n_turns > done:
             _phx.call(L.phx_engine_turns, C.byref(eng), n_turns - done, s)
+
+    def track_turns(self, beam, n_turns, use_graph=True):
+        """Advance beam by n_turns turns."""
+        if n_turns <= 0:
+            return
+        eng = self._prepare(beam, n_turns)
+        s = _phx.stream()
+        done = self._begin(eng, s, use_graph)
+        self._advance(eng, s, n_turns - done, use_graph)
         self._finish(beam)
 
     def timed_turns(self, beam, n_turns):
@@ -550,7 +558,7 @@ class FusedOneTurnMap(Element):
         s = _phx.stream()
         n_st = 3 if self.wake is not None else 1
         first = 3 if eng.ahead else 0
-        n_turns -= self._begin(eng, s, n_turns)
+        n_turns -= self._begin(eng, s, True)
         _phx.call(L.phx_engine_snapshot, C.byref(eng), s)
         ev = [[torch.cuda.Event(enable_timing=True) for _ in range(n_st + 1)]
               for _ in range(n_turns)]
