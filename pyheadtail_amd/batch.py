@@ -47,7 +47,8 @@ class BatchedScan(object):
                                         pass_grid=pass_grid) for m, _ in jobs]
         self.graph_turns = int(graph_turns)
         self.chunk_turns = int(chunk_turns)
-        self._groups = None
+        # the batches by pass variant; those of the turns before programs settle
+        self._groups, self._settling = {}, {}
         self._pass_grid = int(pass_grid)
         self.groups_per_block = 0
         if groups_per_block:
@@ -98,14 +99,14 @@ class BatchedScan(object):
 
     # -- fused mode ----------------------------------------------------------
     def _drop_batches(self):
-        if self._groups:
-            L = _phx.load_library()
-            for grp in self._groups.values():
+        L = _phx.load_library()
+        for groups in (self._groups, self._settling):
+            for grp in groups.values():
                 for h in grp['graphs'].values():
                     L.phx_graph_destroy(h)
                 if grp['batch'] is not None:
                     L.phx_batch_destroy(grp['batch'])
-        self._groups = {}
+        self._groups, self._settling = {}, {}
 
     def __del__(self):
         try:
@@ -114,51 +115,73 @@ class BatchedScan(object):
             pass
 
     def _fused_turns(self, n_turns):
-        L = _phx.lib()
-        s = _phx.stream()
         for eng, b in zip(self.engines, self.bunches):
             eng.reserve(b, max(n_turns, self.graph_turns))
         recs = [eng._prepare(b, n_turns) for eng, b in zip(self.engines, self.bunches)]
-        groups = {}
+        variants = {}
         for i, r in enumerate(recs):
-            # a batch's turns are three launches from the first turn or not
-            if self.engines[i]._unsteady:
-                r.ahead = 0
-            groups.setdefault((r.record_stats, r.program_shape, r.det_shape, r.ahead),
-                              []).append(i)
-        if self._groups is None:
-            self._groups = {}
-        for key, idx in groups.items():
-            arr = (_phx.Engine * len(idx))(*[recs[i] for i in idx])
-            sig = bytes(memoryview(arr).cast("B"))
-            grp = self._groups.get(key)
-            if grp is None or grp['sig'] != sig:
-                if grp is not None:
-                    for h in grp['graphs'].values():
-                        L.phx_graph_destroy(h)
-                    L.phx_batch_destroy(grp['batch'])
-                nb = L.phx_batch_desc_bytes(len(idx))
-                desc = torch.empty(nb, dtype=torch.uint8, device=_phx.device())
-                h = C.c_void_p()
-                _phx.call(L.phx_batch_create, arr, len(idx), desc.data_ptr(), nb, s, C.byref(h))
-                grp = dict(sig=sig, batch=h, desc=desc, arr=arr, graphs={})
-                self._groups[key] = grp
-            G = self.graph_turns
-            done = 0
-            if G > 0 and n_turns >= G:
-                g = grp['graphs'].get(G)
-                if g is None:
-                    g = C.c_void_p()
-                    _phx.call(L.phx_batch_capture, grp['batch'], G, C.byref(g))
-                    grp['graphs'][G] = g
-                _phx.call(L.phx_batch_snapshot, grp['batch'], s)
-                while n_turns - done >= G:
-                    _phx.call(L.phx_graph_launch, g, s)
-                    done += G
-            if n_turns > done:
-                _phx.call(L.phx_batch_turns, grp['batch'], n_turns - done, s)
+            variants.setdefault((r.record_stats, r.program_shape, r.det_shape), []).append(i)
+        for key, idx in variants.items():
+            first = self._three_launch([recs[i] for i in idx], [self.engines[i] for i in idx],
+                                       n_turns)
+            if first:
+                steady = [recs[i].ahead for i in idx]
+                for i in idx:
+                    recs[i].ahead = 0
+                self._advance(self._settling, key, [recs[i] for i in idx], first)
+                for i, ahead in zip(idx, steady):
+                    recs[i].ahead = ahead
+            for ahead in (1, 0):
+                rs = [recs[i] for i in idx if recs[i].ahead == ahead]
+                if rs:
+                    self._advance(self._groups, key + (ahead,), rs, n_turns - first)
         for eng, b in zip(self.engines, self.bunches):
             eng._finish(b)
+
+    @staticmethod
+    def _three_launch(recs, engines, n_turns):
+        """Sets which jobs of a pass variant run three-launch turns (a batch's
+        turns are three launches or not); returns the number of turns that all
+        run in four before, until the last of their programs has settled."""
+        first = max([eng._unsteady for eng, r in zip(engines, recs) if r.ahead] or [0])
+        if n_turns - first < _phx.AHEAD_MIN_TURNS:
+            first = 0
+            for r in recs:
+                r.ahead = 0
+        return first
+
+    def _advance(self, groups, key, recs, n_turns):
+        """n_turns turns of the jobs in one batch, kept in groups[key]."""
+        L = _phx.lib()
+        s = _phx.stream()
+        arr = (_phx.Engine * len(recs))(*recs)
+        sig = bytes(memoryview(arr).cast("B"))
+        grp = groups.get(key)
+        if grp is None or grp['sig'] != sig:
+            if grp is not None:
+                for h in grp['graphs'].values():
+                    L.phx_graph_destroy(h)
+                L.phx_batch_destroy(grp['batch'])
+            nb = L.phx_batch_desc_bytes(len(recs))
+            desc = torch.empty(nb, dtype=torch.uint8, device=_phx.device())
+            h = C.c_void_p()
+            _phx.call(L.phx_batch_create, arr, len(recs), desc.data_ptr(), nb, s, C.byref(h))
+            grp = dict(sig=sig, batch=h, desc=desc, arr=arr, graphs={})
+            groups[key] = grp
+        G = self.graph_turns
+        done = 0
+        if G > 0 and n_turns >= G:
+            g = grp['graphs'].get(G)
+            if g is None:
+                g = C.c_void_p()
+                _phx.call(L.phx_batch_capture, grp['batch'], G, C.byref(g))
+                grp['graphs'][G] = g
+            _phx.call(L.phx_batch_snapshot, grp['batch'], s)
+            while n_turns - done >= G:
+                _phx.call(L.phx_graph_launch, g, s)
+                done += G
+        if n_turns > done:
+            _phx.call(L.phx_batch_turns, grp['batch'], n_turns - done, s)
 
     # -- both modes ----------------------------------------------------------
     def track_turns(self, n_turns):

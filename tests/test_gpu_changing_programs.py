@@ -78,3 +78,70 @@ def test_launch_sequences_and_results(gamma, p_increment, turns, expected, monke
     one, many = to_numpy(one), to_numpy(many)
     for k in COORDS:
         np.testing.assert_array_equal(one[k], many[k], err_msg=k)
+
+
+def _batch_calls(monkeypatch):
+    """[(entry point, ahead of each engine or count of turns)] from here on."""
+    from pyheadtail_amd import _phx
+    seen, call = [], _phx.call
+
+    def counting(fn, *args):
+        name = getattr(fn, "__name__", "")
+        if name == "phx_batch_create":
+            seen.append((name, [args[0][i].ahead for i in range(args[1])]))
+        elif name in ("phx_batch_capture", "phx_batch_turns"):
+            seen.append((name, args[1]))
+        return call(fn, *args)
+    monkeypatch.setattr(_phx, "call", counting)
+    return seen
+
+
+def _alone(jobs, turns):
+    from pyheadtail_amd.engine import FusedOneTurnMap
+    from tests.machines import to_numpy
+    out = []
+    for m, b in jobs:
+        eng = FusedOneTurnMap(m, pass_grid=20, specialise=True)
+        for k in turns:
+            eng.track_turns(b, k, use_graph=False)
+        out.append(to_numpy(b))
+    return out
+
+
+def _check_batch(make, turns, monkeypatch):
+    """The jobs in one scan and each alone, bit for bit; the scan's calls."""
+    from pyheadtail_amd.batch import BatchedScan
+    from tests.machines import COORDS, to_numpy
+    want = _alone(make(), turns)
+    scan = BatchedScan(make(), graph_turns=4, pass_grid=20)
+    seen = _batch_calls(monkeypatch)
+    for k in turns:
+        scan.track_turns(k)
+    for b, w in zip(scan.bunches, want):
+        for k, v in to_numpy(b).items():
+            if k in COORDS:
+                np.testing.assert_array_equal(v, w[k], err_msg=k)
+    return seen
+
+
+def test_scan_with_settling_programs(monkeypatch):
+    """Jobs whose programs settle after 0, 2 and 5 turns: five turns of four
+    launches for all of them, then three-launch turns, in one batch each."""
+    print("\n[case] scan of rings that settle at different turns", flush=True)
+
+    def make():
+        return [(_map(g, 0.), _bunch(g, n, n)) for g, n in ((27.728564, 8000), (11.3, 20011),
+                                                            (50.3, 1025))]
+    seen = _check_batch(make, [14, 9], monkeypatch)
+    assert seen == [("phx_batch_create", [0, 0, 0]), ("phx_batch_capture", 4), ("phx_batch_turns", 1),
+                    ("phx_batch_create", [1, 1, 1]), ("phx_batch_capture", 4), ("phx_batch_turns", 1),
+                    ("phx_batch_turns", 1)]
+
+
+def test_accelerating_scan(monkeypatch):
+    print("\n[case] scan of accelerating rings", flush=True)
+
+    def make():
+        return [(_map(g, 1e-24), _bunch(g, n, n)) for g, n in ((27.728564, 8000), (11.3, 20011))]
+    seen = _check_batch(make, [10], monkeypatch)
+    assert seen == [("phx_batch_create", [0, 0]), ("phx_batch_capture", 4), ("phx_batch_turns", 2)]
