@@ -33,6 +33,16 @@ from .engine import FusedOneTurnMap
 from .serve import job_bytes
 
 
+# Jobs of one pass variant that can run three-launch turns share a batch of
+# four-launch turns with those that cannot (a kick on dp), unless the first
+# hold this many macroparticles together: a second batch is three more
+# launches a turn, the shorter turn gains by the macroparticle.  20 turns, one
+# batch and two: 4 + 4 jobs of 2e4 1106 and 1479 us, of 3e5 2712 and 3000, of
+# 1e6 5171 and 5250, of 1.5e6 7214 and 6639, of 4e6 17041 and 16029; 2 + 2
+# jobs of 1e6 2925 and 3089, of 2e6 4656 and 4648, of 4e6 8923 and 7629.
+MIXED_MIN = 4000000
+
+
 class BatchedScan(object):
 
     def __init__(self, jobs, n_streams=8, chunk_turns=100, graph_turns=10, record_stats=False,
@@ -144,7 +154,9 @@ class BatchedScan(object):
         turns are three launches or not); returns the number of turns that all
         run in four before, until the last of their programs has settled."""
         first = max([eng._unsteady for eng, r in zip(engines, recs) if r.ahead] or [0])
-        if n_turns - first < _phx.AHEAD_MIN_TURNS:
+        n = sum(r.n for r in recs if r.ahead)
+        if (n_turns - first < _phx.AHEAD_MIN_TURNS or
+                (n < MIXED_MIN and not all(r.ahead for r in recs))):
             first = 0
             for r in recs:
                 r.ahead = 0

@@ -145,3 +145,21 @@ def test_accelerating_scan(monkeypatch):
         return [(_map(g, 1e-24), _bunch(g, n, n)) for g, n in ((27.728564, 8000), (11.3, 20011))]
     seen = _check_batch(make, [10], monkeypatch)
     assert seen == [("phx_batch_create", [0, 0]), ("phx_batch_capture", 4), ("phx_batch_turns", 2)]
+
+
+@pytest.mark.parametrize("least,created", [(None, [[0, 0]]), (1, [[1], [0]])])
+def test_scan_with_and_without_kicks_on_dp(least, created, monkeypatch):
+    print("\n[case] scan with and without kicks on dp, least %r" % least, flush=True)
+    from pyheadtail_amd import batch
+    from pyheadtail_amd.impedances.wakes import Resonator, WakeField
+    from pyheadtail_amd.particles.slicing import UniformBinSlicer
+    if least is not None:
+        monkeypatch.setattr(batch, "MIXED_MIN", least)
+
+    def make():
+        jobs = [(_map(27.728564, 0.), _bunch(27.728564, n, n)) for n in (8000, 20011)]
+        jobs[1][0][2] = WakeField(UniformBinSlicer(50, n_sigma_z=3),
+                                  Resonator(1e6, 1e9, 1, 1., 1., 0., 0., True))
+        return jobs
+    seen = _check_batch(make, [9], monkeypatch)
+    assert [v for k, v in seen if k == "phx_batch_create"] == created
