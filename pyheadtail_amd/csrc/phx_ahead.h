@@ -16,6 +16,16 @@ inline size_t ahead_lds_bytes(const phx_engine &e, int nsub) {
          sizeof(double);
 }
 
+// Whether the low limbs of a slice's sums hold what one of the pass's blocks
+// adds to it at most (2^(FX_LB - 1) a particle, below 2^63 together).  Blocks
+// of up to 2^24 particles are every grid's for bunches up to that size, and
+// those of 64 blocks and more for any bunch.
+inline bool ahead_limbs_hold(int64_t n, int grid, int nsub, int hblk) {
+  const int64_t rounds = (grid + (int64_t)hblk * nsub - 1) / ((int64_t)hblk * nsub);
+  const int64_t groups = (phx_n_groups(n) + grid - 1) / grid;
+  return rounds * nsub * groups * PHX_CHUNK <= (1LL << (63 - FX_LB + 1)) - 1;
+}
+
 // Whether the engine's turns can be three launches when e.ahead is set.
 bool ahead_fits(const phx_engine &e);
 // Groups of threads per block of its pass.

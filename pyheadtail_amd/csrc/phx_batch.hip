@@ -431,6 +431,7 @@ extern "C" int phx_batch_create(const phx_engine *engines, int32_t n, void *desc
       const int hb = hist_blocks(e.n);
       a.hblk = (a.grid + PHX_BATCH_NSUB - 1) / PHX_BATCH_NSUB;
       a.hblk = a.hblk < hb ? a.hblk : hb;
+      B->ahead = B->ahead && ahead_limbs_hold(e.n, a.grid, PHX_BATCH_NSUB, a.hblk);
       const size_t la = ahead_lds_bytes(e, PHX_BATCH_NSUB);
       B->lds_ahead = la > B->lds_ahead ? la : B->lds_ahead;
     }

@@ -452,6 +452,7 @@ EngineArgs make_args(const phx_engine *e, int nk, int T) {
     a.hblk = (a.grid + a.nsub - 1) / a.nsub;
     const int hb = hist_blocks(e->n);
     a.hblk = a.hblk < hb ? a.hblk : hb;
+    if (!ahead_limbs_hold(e->n, a.grid, a.nsub, a.hblk)) a.nsub = a.hblk = 0;
   }
   return a;
 }
