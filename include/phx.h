@@ -692,6 +692,9 @@ int phx_engine_reset(const phx_engine *e, phx_stream_t stream);
    its cuts.  The results are those of the four-launch turn bit for bit. */
 #define PHX_AHEAD_MIN_TURNS 4
 int phx_engine_turns(const phx_engine *e, int32_t n_turns, phx_stream_t stream);
+/* 1 if phx_engine_turns(e, n_turns, ...) runs three-launch turns, 0 if not (or
+   an error code). */
+int phx_engine_three_launch(const phx_engine *e, int32_t n_turns);
 /* Applies a pending wake kick (and records the final statistics row). */
 int phx_engine_flush(const phx_engine *e, phx_stream_t stream);
 /* Enqueue one stage of a turn: 0 particle pass, 1 slice histogram and
@@ -748,6 +751,9 @@ int64_t phx_batch_desc_bytes(int32_t n);
 int phx_batch_create(const phx_engine *engines, int32_t n, void *desc, int64_t desc_bytes,
                      phx_stream_t stream, void **batch);
 int phx_batch_turns(void *batch, int32_t n_turns, phx_stream_t stream);
+/* 1 if phx_batch_turns(batch, n_turns, ...) runs three-launch turns, 0 if not
+   (or an error code). */
+int phx_batch_three_launch(void *batch, int32_t n_turns);
 int phx_batch_snapshot(void *batch, phx_stream_t stream);
 int phx_batch_capture(void *batch, int32_t n_turns, void **graph);
 int phx_batch_destroy(void *batch);

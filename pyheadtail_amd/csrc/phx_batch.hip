@@ -361,8 +361,12 @@ int batch_begin(const Batch &B, bool ahead, hipStream_t s) {
   return PHX_OK;
 }
 
+bool batch_three_launch(const Batch &B, int n_turns, bool snapshot) {
+  return B.ahead && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
+}
+
 int batch_turns(const Batch &B, int n_turns, hipStream_t s, bool snapshot) {
-  const bool ahead = B.ahead && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
+  const bool ahead = batch_three_launch(B, n_turns, snapshot);
   if (snapshot && n_turns > 0) {
     const int rc = batch_begin(B, ahead, s);
     if (rc) return rc;
@@ -474,6 +478,11 @@ extern "C" int phx_batch_turns(void *batch, int32_t n_turns, phx_stream_t stream
   if (!batch) return phx::fail(PHX_E_INVALID, "phx_batch_turns: null batch");
   if (n_turns < 0) return phx::fail(PHX_E_INVALID, "phx_batch_turns: n_turns < 0");
   return batch_turns(*reinterpret_cast<Batch *>(batch), n_turns, phx::as_stream(stream), true);
+}
+
+extern "C" int phx_batch_three_launch(void *batch, int32_t n_turns) {
+  if (!batch) return phx::fail(PHX_E_INVALID, "phx_batch_three_launch: null batch");
+  return batch_three_launch(*reinterpret_cast<Batch *>(batch), n_turns, true) ? 1 : 0;
 }
 
 extern "C" int phx_batch_snapshot(void *batch, phx_stream_t stream) {

@@ -654,10 +654,17 @@ extern "C" int phx_engine_reset(const phx_engine *e, phx_stream_t stream) {
   return PHX_OK;
 }
 
-// n_turns turns, after a snapshot of particle 0 (and, for three-launch turns,
-// their start) if snapshot is set.  A sequence without one continues another
-// that had it.  The start costs two launches and a read of x, y, z and dp
-// (13 us at 1e6 macroparticles), less than PHX_AHEAD_MIN_TURNS turns gain.
+// Whether n_turns turns are three launches each.  The start of a sequence costs
+// two launches and a read of x, y, z and dp (1e6 macroparticles: 13.6 + 8.1 us
+// against 2 us for the snapshot), less than PHX_AHEAD_MIN_TURNS turns gain (7 us
+// each at 1e4, 8 us at 1e6, 43 us at 1e7 macroparticles).  A sequence without a
+// snapshot continues another that had the start.
+static bool three_launch(const EngineArgs &a, int32_t n_turns, bool snapshot) {
+  return a.nsub > 0 && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
+}
+
+// n_turns turns, after a snapshot of particle 0 (for three-launch turns, after
+// their start) if snapshot is set.
 static int engine_turns(const phx_engine *e, int32_t n_turns, hipStream_t s, bool snapshot) {
   int nk, T;
   int rc = check_engine(e, &nk, &T);
@@ -667,7 +674,7 @@ static int engine_turns(const phx_engine *e, int32_t n_turns, hipStream_t s, boo
   if (rc) return rc;
   const bool has_wake = e->n_slices > 0 && nk > 0;
   EngineArgs a = make_args(e, nk, T);
-  const bool ahead = a.nsub > 0 && (!snapshot || n_turns >= PHX_AHEAD_MIN_TURNS);
+  const bool ahead = three_launch(a, n_turns, snapshot);
   if (snapshot && n_turns > 0) {
     rc = ahead ? ahead_enqueue_start(a, s) : enqueue_snapshot(a, s);
     if (rc) return rc;
@@ -681,6 +688,12 @@ static int engine_turns(const phx_engine *e, int32_t n_turns, hipStream_t s, boo
 
 extern "C" int phx_engine_turns(const phx_engine *e, int32_t n_turns, phx_stream_t stream) {
   return engine_turns(e, n_turns, phx::as_stream(stream), true);
+}
+
+extern "C" int phx_engine_three_launch(const phx_engine *e, int32_t n_turns) {
+  EngineArgs a;
+  const int rc = engine_args_for(e, &a);
+  return rc ? rc : (three_launch(a, n_turns, true) ? 1 : 0);
 }
 
 extern "C" int phx_engine_stage(const phx_engine *e, int32_t stage, phx_stream_t stream) {
