@@ -689,7 +689,12 @@ int phx_engine_reset(const phx_engine *e, phx_stream_t stream);
    when it starts, slices the particles it has just moved, and sums the next
    turn's z (the longitudinal motion alone fixes it) for the next turn's
    cuts, which the merge folds.  Two launches ahead of the first turn give
-   its cuts.  The results are those of the four-launch turn bit for bit. */
+   its cuts.  The results are those of the four-launch turn bit for bit,
+   except where the scale of a turn's slice sums differs: it comes from the
+   largest |x|, |y| of the state before the turn here and after it there, as
+   2^P with P the multiple of 8 at or above ilogb + 2 of it.  If the two lie on
+   either side of a step of P, a value is kept to 2^(P - 74) with either P,
+   which shows in the last bits of slices of few macroparticles. */
 #define PHX_AHEAD_MIN_TURNS 4
 int phx_engine_turns(const phx_engine *e, int32_t n_turns, phx_stream_t stream);
 /* 1 if phx_engine_turns(e, n_turns, ...) runs three-launch turns, 0 if not (or

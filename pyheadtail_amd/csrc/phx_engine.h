@@ -612,8 +612,10 @@ __device__ __forceinline__ void pass_body(
 // the longitudinal motion (nothing for a linear map, a sine for an RF kick).
 // One pass block is nsub groups of PHX_BLOCK threads, each a block of the
 // four-launch pass (the same particles in the same order, hence the same z
-// sums, cuts and coordinates bit for bit), sharing one histogram: a CU then
-// stores one partial histogram, as many as the histogram kernel stored.
+// sums and cuts bit for bit), sharing one histogram: a CU then stores one
+// partial histogram, as many as the histogram kernel stored.  The slices' sums
+// are the four-launch turn's too unless the bounds of |x| and |y|, which are
+// those of the state before the turn, give them another scale (fx_scale).
 // ---------------------------------------------------------------------------
 __host__ __device__ inline size_t ahead_hist_doubles(int S) {
   return (acc_lds_bytes(S, 2) + 7) / 8;
