@@ -689,8 +689,10 @@ def headline_turns(n, args, steps, stage_turns):
     # buffers for the longest call, so that no later call re-allocates them
     # or captures its graph again
     eng.reserve(bunch, max(steps, stage_turns, args.warmup, args.graph_turns))
-    # warm-up (the graph is captured here)
+    # warm-up, then the turns that capture the graph: p0's last bit moves in an
+    # RF ring's first turns, which are launched one by one
     eng.track_turns(bunch, max(args.warmup, args.graph_turns))
+    eng.track_turns(bunch, args.graph_turns)
     bunch.x  # applies the pending kick
     torch.cuda.synchronize()
     # per-stage kernel durations with HIP events on the launch stream
