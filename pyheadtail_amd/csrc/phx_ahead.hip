@@ -8,7 +8,7 @@ using namespace phx_en;
 namespace {
 
 template <bool REC, int SHAPE, int KS, int DS>
-__global__ void __launch_bounds__((ahead_nsub<REC, SHAPE>() * PHX_BLOCK))
+__global__ void __launch_bounds__((ahead_nsub<REC, SHAPE, DS>() * PHX_BLOCK))
     k_engine_ahead(EngineArgs a, double *__restrict__ x, double *__restrict__ xp,
                    double *__restrict__ y, double *__restrict__ yp, double *__restrict__ z,
                    double *__restrict__ dp, const phx_turn_program *__restrict__ programs,
@@ -39,22 +39,26 @@ void launch(const EngineArgs &a, hipStream_t s) {
           a, c[0], c[1], c[2], c[3], c[4], c[5], e.programs, e.kicks);
 }
 
+template <bool REC, int SHAPE, int KS, int DS>
+AheadPass compiled() {
+  return {launch<REC, SHAPE, KS, DS>, ahead_nsub<REC, SHAPE, DS>()};
+}
+
 template <bool REC, int SHAPE, int KS>
 AheadPass pick_dets(int ds) {
-  constexpr int NS = ahead_nsub<REC, SHAPE>();
   if constexpr (!REC && SHAPE != PHX_SHAPE_GENERIC) {
     switch (ds) {
-      case PHX_DETS_NONE: return {launch<REC, SHAPE, KS, PHX_DETS_NONE>, NS};
-      case PHX_DETS_C1: return {launch<REC, SHAPE, KS, PHX_DETS_C1>, NS};
-      case PHX_DETS_C1_AMP: return {launch<REC, SHAPE, KS, PHX_DETS_C1_AMP>, NS};
+      case PHX_DETS_NONE: return compiled<REC, SHAPE, KS, PHX_DETS_NONE>();
+      case PHX_DETS_C1: return compiled<REC, SHAPE, KS, PHX_DETS_C1>();
+      case PHX_DETS_C1_AMP: return compiled<REC, SHAPE, KS, PHX_DETS_C1_AMP>();
       case PHX_DETS_C1 | PHX_DETS_SMOOTH:
-        return {launch<REC, SHAPE, KS, PHX_DETS_C1 | PHX_DETS_SMOOTH>, NS};
+        return compiled<REC, SHAPE, KS, PHX_DETS_C1 | PHX_DETS_SMOOTH>();
       case PHX_DETS_C1_AMP | PHX_DETS_SMOOTH:
-        return {launch<REC, SHAPE, KS, PHX_DETS_C1_AMP | PHX_DETS_SMOOTH>, NS};
+        return compiled<REC, SHAPE, KS, PHX_DETS_C1_AMP | PHX_DETS_SMOOTH>();
       default: break;
     }
   }
-  return {launch<REC, SHAPE, KS, PHX_DETS_GENERIC>, NS};
+  return compiled<REC, SHAPE, KS, PHX_DETS_GENERIC>();
 }
 
 template <bool REC, int KS>

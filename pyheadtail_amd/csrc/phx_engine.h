@@ -633,10 +633,19 @@ __host__ __device__ constexpr int ahead_red_doubles() {
   return REC ? BR_LDS(EN_STAT_NV) : BR_LDS(ZA_NV);
 }
 // Groups of threads per block: three of the specialised passes' groups fill a
-// CU (at most 168 vector registers), two of the others'.
-template <bool REC, int SHAPE>
+// CU (at most 168 vector registers), two of the others'.  Two-harmonic RF with
+// amplitude detuning takes two: in 168 registers it spills 4 to 22 of them (40
+// turns of 3e5, of 1e6 and 10 turns of 5e6 macroparticles, three and two
+// groups: 1152 and 967, 1864 and 1572, 1485 and 1207 us); with chromaticity
+// alone it spills 4 to 13 and keeps three (1015 and 945, 1532 and 1531, 1143
+// and 1167 us).  The generic order with statistics spills at two as well; one
+// group is the better up to 3e5 macroparticles (40 turns 2002 against 2204 us),
+// two above (1e6: 3677 against 3589, 10 turns of 5e6: 3517 against 3079).
+template <bool REC, int SHAPE, int DS>
 constexpr int ahead_nsub() {
-  return REC || SHAPE == PHX_SHAPE_GENERIC ? 2 : 3;
+  constexpr bool RF2 = SHAPE == PHX_SHAPE_RF2_T || SHAPE == PHX_SHAPE_T_RF2;
+  constexpr bool AMP = (DS & ~PHX_DETS_SMOOTH) == PHX_DETS_C1_AMP;
+  return REC || SHAPE == PHX_SHAPE_GENERIC || (RF2 && AMP) ? 2 : 3;
 }
 
 // The partial histograms of a three-launch turn: hblk of them, the fallback
