@@ -269,13 +269,13 @@ typedef struct {
     double beta_ratio, eta0, length;
     /* kick: phi = (h*((2pi*z)/C) + phi_offset) + phi_lock
              dp <- (dp*p0_before + ((amplitude*sin(phi)) - p_increment))
-                   / p0_after                               (:195-203) */
+                   / p0_after                               (:195-203)
+       evaluated with phi in turns and the quotients by C and p0_after folded
+       into the kick's constants */
     double harmonic, two_pi, circumference, phi_offset, phi_lock;
     double amplitude, p_increment, p0_before, p0_after;
     double D_x, D_y;
-    /* 1.0 / circumference and 1.0 / p0_after (IEEE divisions): the kick's
-       two divisions are formed from them and rounded exactly as the
-       divisions themselves */
+    /* 1.0 / circumference and 1.0 / p0_after (IEEE divisions) */
     double inv_circumference, inv_p0_after;
 } phx_long_op;
 
@@ -319,12 +319,12 @@ typedef struct {
 int phx_transverse_damper(double *xp, double *yp, int64_t n, const double *sums,
                           const phx_damper *p, phx_stream_t stream);
 
-/* The FP64 sine and cosine the maps evaluate on the device (the detuned
-   betatron phase, the RF phase): s[i] = sin(x[i]), c[i] = cos(x[i]) for
-   device arrays of n values; either output may be null.  No reference
-   counterpart: it exposes the device arithmetic behind
-   TransverseSegmentMap.track and Kick.track (np.sin / np.cos,
-   general/pmath.py:178-179, 239) for accuracy checks. */
+/* The FP64 sine and cosine of an argument in radians that the wake functions
+   evaluate on the device: s[i] = sin(x[i]), c[i] = cos(x[i]) for device
+   arrays of n values; either output may be null.  (The maps count their
+   phases in turns and form theirs from those.)  No reference counterpart: it
+   exposes the device arithmetic behind np.sin / np.cos
+   (general/pmath.py:178-179, 239) for accuracy checks. */
 int phx_math_sincos(const double *x, int64_t n, double *s, double *c,
                     phx_stream_t stream);
 
